@@ -76,7 +76,7 @@ double uniform01(uint64_t seed, uint64_t counter) {
 int64_t run_bytes(const Geom& g, int phys, int prec) {
   const int s = prec == 0 ? 4 : 8;
   const int nf = phys == PHYS_MHD ? 6 : 3;
-  const int np = phys == PHYS_MHD ? 9 : 6;
+  const int np = work_fields(phys);
   const int64_t rows = (int64_t)g.ny * g.nz;
   const int64_t blocks = prec == 0 ? row_blocks_max<float>(g.nx, rows) : row_blocks_max<double>(g.nx, rows);
   return (int64_t)(3 * nf) * g.nc * 2 * s + (int64_t)np * g.wnc * 2 * s + (int64_t)nf * g.nr * s + 2 * blocks * s +
@@ -87,7 +87,7 @@ template <class T>
 class Engine : public EngineBase {
  public:
   Geom g{};
-  int phys = 0, nf = 0, np = 0, stepper = 0, nr_ = 0, dev = 0;
+  int phys = 0, nf = 0, np = 0 /* advective products without modules */, stepper = 0, nr_ = 0, dev = 0;
   hipStream_t st = nullptr;
   // Second stream and events of the slab pipeline (see rhs), and the stream the hot launches
   // go to (st, or st2 for odd slabs).
@@ -98,7 +98,7 @@ class Engine : public EngineBase {
   RunBuf<T>* rbd = nullptr;
   std::vector<void*> allocs;
   std::vector<RunClock> clk_init;
-  const cx<T>*twy = nullptr, *twz = nullptr, *twM = nullptr, *twh = nullptr;
+  const cx<T>*twy = nullptr, *twz = nullptr, *twM = nullptr, *twh = nullptr, *twx = nullptr;
   int64_t row_blocks = 0;
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -157,7 +157,7 @@ class Engine : public EngineBase {
     lens[2] = L[2];
     phys = ph;
     nf = ph == PHYS_MHD ? 6 : 3;
-    np = ph == PHYS_MHD ? 9 : 6;
+    np = nadv(ph);
     stepper = stp;
     nr_ = (int)rp.size();
     dev = device;
@@ -184,6 +184,7 @@ class Engine : public EngineBase {
     int err = 0;
     twy = twiddles<T>(device, g.ny, 0, &err);
     twz = twiddles<T>(device, g.nz, 0, &err);
+    twx = twiddles<T>(device, g.nx, 0, &err);
     twM = twiddles<T>(device, g.nx / 2, 0, &err);
     twh = twiddles<T>(device, g.nx, 1, &err);
     if (err) return err;
@@ -195,7 +196,7 @@ class Engine : public EngineBase {
     ndf_bufs.assign(nr_, nullptr);
     ndpart_bufs.assign(nr_, nullptr);
     vp_bufs.assign(nr_, nullptr);
-    np_alloc = np;
+    np_alloc = work_fields(phys);
     for (int r = 0; r < nr_; ++r) {
       RunBuf<T>& b = rbh[r];
       std::memset(&b, 0, sizeof(b));
@@ -213,7 +214,7 @@ class Engine : public EngineBase {
       b.rscr = (T*)p;
       MHD_TRY(alloc(cb * nf, &p));
       b.buf[B_ACC] = (cx<T>*)p;
-      MHD_TRY(alloc(sizeof(cx<T>) * (size_t)g.wnc * np, &p));
+      MHD_TRY(alloc(sizeof(cx<T>) * (size_t)g.wnc * np_alloc, &p));
       b.buf[B_WORK] = (cx<T>*)p;
       MHD_TRY(alloc(sizeof(T) * (size_t)g.nr * nf, &p));
       b.vars = (T*)p;
@@ -288,7 +289,7 @@ class Engine : public EngineBase {
   // block); returns the number of slabs, 1 when the pipeline is off
   int pipe_slabs(int rvar, std::vector<int>* zb) const {
     if (pipe_ <= 1 || rec_ || profiling || nd_any || vp_any) return 1;
-    const int rpb = row_rows_per_block<T>(g.nx, rvar);
+    const int rpb = rhs_rows_per_block(rvar);
     int q = 1;  // z-planes per row-block boundary: q*ny is a multiple of rpb
     while ((int64_t)q * g.ny % rpb) ++q;
     zb->assign(1, 0);
@@ -393,23 +394,38 @@ class Engine : public EngineBase {
     return timed(name, bytes, [&] { return launch_colpass<T>(a, n, dir, S, cur_rb(), tw, cs_); });
   }
 
-  // row launches: variant 0 everywhere except the fused products kernel (row_var)
-  RowArgs row_args(int var = 0) const {
+  // The fused row launch of a right-hand side: rowpair_kernel, or xrow_kernel for runs with a
+  // calcF! module or volume penalisation.  Variant row_var: of xrow_kernel as it is; for
+  // rowpair_kernel bit 0 picks the plan that rowpair_plan does not.
+  bool row_pairs() const { return !active_module(); }
+  int rhs_rows_per_block(int var) const {
+    return row_pairs() ? rowpair_rows_per_block(g.nx, var) : row_rows_per_block<T>(g.nx, var);
+  }
+  int rhs_row_variant() const { return row_pairs() ? rowpair_plan(g.nx, phys) ^ (row_var & 1) : row_var; }
+  RowArgs rhs_row_args(int var) const { return row_args_of(rhs_rows_per_block(var)); }
+  // the other row launches: xrow_kernel, variant 0
+  RowArgs row_args() const { return row_args_of(row_rows_per_block<T>(g.nx)); }
+  RowArgs row_args_of(int64_t rpb) const {
     RowArgs r{};
     r.g = g;
     r.nruns = cur_n();
     r.rows = (int64_t)g.ny * g.nz;
-    const int64_t rpb = row_rows_per_block<T>(g.nx, var);
     r.blocks_per_run = (r.rows + rpb - 1) / rpb;
     r.in_ncols = g.nkr;
     r.gate = gate_;
     return r;
   }
 
-  int xrow(const char* name, const RowArgs& a, int kind, int nfk, double bytes, int var = 0) {
+  hipError_t launch_row(const RowArgs& a, int kind, int nfk, int var, bool pairs, const RunBuf<T>* runs,
+                        hipStream_t s) {
+    return pairs ? launch_rowpair<T>(a, kind, var, runs, twx, s) : launch_xrow<T>(a, kind, nfk, var, runs, twM, twh, s);
+  }
+
+  int xrow(const char* name, const RowArgs& a, int kind, int nfk, double bytes, int var = 0, bool pairs = false) {
     if (rec_) {
       Rec r;
       r.type = Rec::ROW;
+      r.pairs = pairs;
       r.n = g.nx;
       r.kind = kind;
       r.var = var;
@@ -419,7 +435,7 @@ class Engine : public EngineBase {
       rec_->push_back(r);
       return 0;
     }
-    return timed(name, bytes, [&] { return launch_xrow<T>(a, kind, nfk, var, cur_rb(), twM, twh, cs_); });
+    return timed(name, bytes, [&] { return launch_row(a, kind, nfk, var, pairs, cur_rb(), cs_); });
   }
 
   // A launch that is not one of the hot kinds: run now, or recorded as a closure over the
@@ -439,12 +455,13 @@ class Engine : public EngineBase {
   // ---- recording of a time step for multi-size ensemble launches -----------------
   // While rec_ is set, step_launches_gated() records the hot launches with their arguments
   // instead of launching them, and the other launches as closures.  With rec_multi_ the
-  // shapes are the multi-size kernels' (column strips of 128 threads, the row plan without
-  // the LDS swizzle); otherwise the group's own tuned shapes.
+  // shapes are the multi-size kernels' (column strips of 128 threads); otherwise the group's own
+  // tuned shapes.
   struct Rec {
     enum { OTHER = 0, COL = 1, ROW = 2, SPEC = 3 };
     int type = OTHER;
     int n = 0, dir = 0, kind = 0, var = 0, S = 0, nfk = 0;
+    bool pairs = false;  // a ROW launch of rowpair_kernel
     ColArgs ca{};
     RowArgs ra{};
     SpecArgs sa{};
@@ -470,7 +487,7 @@ class Engine : public EngineBase {
   hipError_t launch_rec(const Rec& r, hipStream_t s) {
     switch (r.type) {
       case Rec::COL: return launch_colpass<T>(r.ca, r.n, r.dir, r.S, r.runs, r.tw, s);
-      case Rec::ROW: return launch_xrow<T>(r.ra, r.kind, r.nfk, r.var, r.runs, twM, twh, s);
+      case Rec::ROW: return launch_row(r.ra, r.kind, r.nfk, r.var, r.pairs, r.runs, s);
       case Rec::SPEC: return launch_spectral<T>(r.sa, phys, r.runs, s);
       default: return r.fn(s);
     }
@@ -538,13 +555,13 @@ class Engine : public EngineBase {
         rc = colpass("tune", 2, 1, B_SOL, B_WORK, 0, 0, nf, true, true);
         if (rc == 0) rc = colpass("tune", 1, 1, B_WORK, B_WORK, 0, 0, nf, true, true);
         if (rc) break;
-        RowArgs ra = row_args(row_var);
+        RowArgs ra = rhs_row_args(rhs_row_variant());
         ra.prune_out = gate_;
         ra.in_sel = B_WORK;
         ra.in_ncols = g.kx_keep;
         ra.out_sel = B_WORK;
         MHD_HIP(hipEventRecord(a, st));
-        rc = xrow("tune", ra, phys == PHYS_MHD ? ROW_MHD : ROW_HD, nf, 0, row_var);
+        rc = xrow("tune", ra, phys == PHYS_MHD ? ROW_MHD : ROW_HD, nf, 0, rhs_row_variant(), row_pairs());
         MHD_HIP(hipEventRecord(b, st));
         MHD_HIP(hipEventSynchronize(b));
         float e = 0;
@@ -560,15 +577,7 @@ class Engine : public EngineBase {
         case 0: rc = colpass("tune", 2, 1, B_SOL, B_WORK, 0, 0, nf, true, true); break;
         case 1: rc = colpass("tune", 1, 1, B_WORK, B_WORK, 0, 0, nf, true, true); break;
         case 2: rc = colpass("tune", 1, -1, B_WORK, B_WORK, 0, 0, np, false, true, false, gate_ != 0); break;
-        case 3: rc = colpass("tune", 2, -1, B_WORK, B_WORK, 0, 0, np, false, true, false, gate_ != 0); break;
-        default: {
-          RowArgs ra = row_args(row_var);
-          ra.prune_out = gate_;
-          ra.in_sel = B_WORK;
-          ra.in_ncols = g.kx_keep;
-          ra.out_sel = B_WORK;
-          rc = xrow("tune", ra, phys == PHYS_MHD ? ROW_MHD : ROW_HD, nf, 0, row_var);
-        }
+        default: rc = colpass("tune", 2, -1, B_WORK, B_WORK, 0, 0, np, false, true, false, gate_ != 0); break;
       }
     }
     MHD_HIP(hipEventRecord(b, st));
@@ -600,10 +609,11 @@ class Engine : public EngineBase {
             if (col_strip<T>(n, u) == col_strip<T>(n, v)) dup = true;
           if (dup) continue;
         } else {
-          // row variants: bit 0 plan, bit 1 swizzled LDS; skip a plan equal to a lower variant's
-          bool dup = false;
+          // xrow_kernel: bit 0 plan, bit 1 swizzled LDS; skip a plan equal to a lower variant's.
+          // rowpair_kernel: bit 0 plan
+          bool dup = row_pairs() && v > 1;
           for (int u = 0; u < v; ++u)
-            if ((u >> 1) == (v >> 1) && row_rows_per_block<T>(g.nx, u) == row_rows_per_block<T>(g.nx, v)) dup = true;
+            if (!row_pairs() && (u >> 1) == (v >> 1) && row_rows_per_block<T>(g.nx, u) == row_rows_per_block<T>(g.nx, v)) dup = true;
           if (dup) continue;
         }
         float ms = 0;
@@ -674,11 +684,11 @@ class Engine : public EngineBase {
     // volume penalisation adds nf products chi/eta (v - V0) (u, and b for MHD) to every one
     const bool nd = nd_any && phys == PHYS_MHD && sp.add_force;
     const bool vp = vp_any;
-    // a recorded step keeps the row plan (variant bit 0) and drops the LDS swizzle (bit 1),
-    // which the multi-size row kernel does not have and which changes no value
-    const int rvar = (nd || vp) ? 0 : ((rec_ && rec_multi_) ? (row_var & 1) : row_var);
-    const int npf = nd ? 12 : (vp ? np + nf : np);
-    RowArgs ra = row_args(rvar);
+    const bool pairs = row_pairs();
+    const int rvar = (nd || vp) ? 0 : rhs_row_variant();
+    const int nprod = pairs ? np : nprod_all(phys);
+    const int npf = nd ? nprod + 3 : (vp ? nprod + nf : nprod);
+    RowArgs ra = rhs_row_args(rvar);
     ra.in_sel = B_WORK;
     ra.in_ncols = prune ? g.kx_keep : g.nkr;
     ra.out_sel = B_WORK;
@@ -696,7 +706,7 @@ class Engine : public EngineBase {
     const int nslab = pipe_slabs(rvar, &zb);
     if (nslab <= 1) {
       MHD_TRY(colpass("ypass_inv", 1, 1, B_WORK, B_WORK, 0, 0, nf, prune, true));
-      MHD_TRY(xrow("xrow_fused", ra, kind, nf, bytes, rvar));
+      MHD_TRY(xrow("xrow_fused", ra, kind, nf, bytes, rvar, pairs));
       MHD_TRY(colpass("ypass_fwd", 1, -1, B_WORK, B_WORK, 0, 0, npf, false, true, false, gate_ != 0));
     } else {
       struct SlabReset {  // back to the whole grid on st on every return path
@@ -707,7 +717,7 @@ class Engine : public EngineBase {
           e->slab_z1_ = -1;
         }
       } reset{this};
-      const int64_t rpb = row_rows_per_block<T>(g.nx, rvar);
+      const int64_t rpb = rhs_rows_per_block(rvar);
       MHD_HIP(hipEventRecord(ev_fork, st));
       MHD_HIP(hipStreamWaitEvent(st2, ev_fork, 0));
       for (int k = 0; k < nslab; ++k) {
@@ -719,7 +729,7 @@ class Engine : public EngineBase {
         rs.blk0 = (int64_t)slab_z0_ * g.ny / rpb;
         rs.rows = (int64_t)slab_z1_ * g.ny;
         rs.blocks_per_run = (rs.rows - rs.blk0 * rpb + rpb - 1) / rpb;
-        MHD_TRY(xrow("xrow_fused", rs, kind, nf, bytes * (slab_z1_ - slab_z0_) / g.nz, rvar));
+        MHD_TRY(xrow("xrow_fused", rs, kind, nf, bytes * (slab_z1_ - slab_z0_) / g.nz, rvar, pairs));
         MHD_TRY(colpass("ypass_fwd", 1, -1, B_WORK, B_WORK, 0, 0, npf, false, true, false, gate_ != 0));
       }
       MHD_HIP(hipEventRecord(ev_join, st2));
@@ -758,7 +768,7 @@ class Engine : public EngineBase {
     const double c = sizeof(cx<T>) * (double)nr_;
     const double kept = (double)g.kx_keep * nkept_y(g) * nkept_z(g);
     const double all = (sp.gate && host_pruned_) ? kept : (double)g.nc;  // pruned step: kept modes only
-    double rd = (np + forcing_fields()) * all, wr = 0;
+    double rd = ((row_pairs() ? np : nprod_all(phys)) + forcing_fields()) * all, wr = 0;
     if (sp.mode == SP_RK4) {
       rd += nf * kept;                                  // stage input
       if (sp.stage > 0) rd += nf * kept + nf * all;     // base sol + acc
@@ -788,10 +798,13 @@ class Engine : public EngineBase {
     return false;
   }
 
+  // a module that acts on the right-hand side (HD discards the forcing modules)
+  bool active_module() const { return phys == PHYS_MHD ? any_module() : vp_any; }
+
   SpecArgs spec_base() const {
     SpecArgs s{};
     s.g = g;
-    s.modules = any_module() ? 1 : 0;
+    s.modules = active_module() ? 1 : 0;
     s.mask_input = 1;
     s.add_force = 1;
     s.self_sel = -1;
@@ -1152,11 +1165,12 @@ class Engine : public EngineBase {
     ra.out2_sel = B_STIN;
     ra.out2_f0 = 0;
     MHD_TRY(xrow("xrow_vars", ra, phys == PHYS_MHD ? ROW_VARS_MHD : ROW_VARS_HD, nf, 0));
-    MHD_TRY(colpass("ypass_fwd", 1, -1, B_WORK, B_WORK, 0, 0, np, false));
-    MHD_TRY(colpass("zpass_fwd", 2, -1, B_WORK, B_WORK, 0, 0, np, false));
+    MHD_TRY(colpass("ypass_fwd", 1, -1, B_WORK, B_WORK, 0, 0, nprod_all(phys), false));
+    MHD_TRY(colpass("zpass_fwd", 2, -1, B_WORK, B_WORK, 0, 0, nprod_all(phys), false));
     MHD_TRY(colpass("ypass_fwd", 1, -1, B_STIN, B_STIN, 0, 0, nf, false));
     MHD_TRY(colpass("zpass_fwd", 2, -1, B_STIN, B_STIN, 0, 0, nf, false));
     SpecArgs sp = spec_base();
+    sp.modules = 1;  // the instance that reads xrow_item's products
     sp.nruns = 1;
     sp.nitems = g.nc;
     sp.mode = SP_RHS;
@@ -1642,7 +1656,7 @@ class Engine : public EngineBase {
     }
     MHD_TRY(device_alloc(sizeof(double) * (size_t)row_blocks, &d));
     ndpart_bufs[run] = d;
-    if (phys == PHYS_MHD) MHD_TRY(grow_work(run, 12));  // room for the three f_i u_i products
+    if (phys == PHYS_MHD) MHD_TRY(grow_work(run, nprod_all(phys) + 3));  // room for the three f_i u_i products
     b.ndf = (const T*)ndf_bufs[run];
     b.ndpart = (double*)ndpart_bufs[run];
     b.nd_P = P;
@@ -1697,7 +1711,7 @@ class Engine : public EngineBase {
       if (phys == PHYS_MHD && B0 && B0[c])
         MHD_HIP(hipMemcpyAsync(base + (4 + c) * (size_t)g.nr, B0[c], fb, hipMemcpyHostToDevice, st));
     }
-    MHD_TRY(grow_work(run, np + nf));
+    MHD_TRY(grow_work(run, nprod_all(phys) + nf));
     b.vp = base;
     vp_any = true;
     drop_graph();
@@ -1954,7 +1968,7 @@ class FusedStep : public FusedBase {
     for (int pv = 0; pv < 2; ++pv) {
       std::vector<int> sel;
       for (int k = 0; k < ng_all; ++k)
-        if (type != Rec::ROW || (recm[k][i].var & 1) == pv) sel.push_back(k);
+        if (type != Rec::ROW || recm[k][i].var == pv) sel.push_back(k);
       for (size_t c0 = 0; c0 < sel.size(); c0 += MULTI_MAX) {
         const int ng = (int)std::min<size_t>(MULTI_MAX, sel.size() - c0);
         hipError_t e = hipSuccess;
@@ -1979,8 +1993,7 @@ class FusedStep : public FusedBase {
             m.nx[j] = r.n;
             m.a[j] = r.ra;
             m.runs[j] = r.runs;
-            m.twM[j] = es[k]->twM;
-            m.twh[j] = es[k]->twh;
+            m.twx[j] = es[k]->twx;
             m.start[j + 1] = m.start[j] + r.ra.blocks_per_run * r.ra.nruns;
           }
           e = launch_xrow_multi<T>(m, recm[sel[c0]][i].kind, pv, s);

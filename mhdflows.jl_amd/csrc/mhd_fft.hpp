@@ -133,6 +133,28 @@ template <class T, int S> struct Bfly<T, 6, S> {
   }
 };
 
+template <class T, int S> struct Bfly<T, 12, S> {
+  static __device__ __forceinline__ void run(cx<T>* x) {
+    // 12 = 3 x 4, coprime factors: inputs n = 4 n1 + 3 n2, outputs k = 4 k1 + 9 k2 (mod 12), no
+    // twiddles in between (Good 1958)
+    cx<T> a[4][3];
+#pragma unroll
+    for (int n2 = 0; n2 < 4; ++n2) {
+      cx<T> v[3] = {x[3 * n2 % 12], x[(4 + 3 * n2) % 12], x[(8 + 3 * n2) % 12]};
+      Bfly<T, 3, S>::run(v);
+#pragma unroll
+      for (int k1 = 0; k1 < 3; ++k1) a[n2][k1] = v[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+      cx<T> v[4] = {a[0][k1], a[1][k1], a[2][k1], a[3][k1]};
+      Bfly<T, 4, S>::run(v);
+#pragma unroll
+      for (int k2 = 0; k2 < 4; ++k2) x[(4 * k1 + 9 * k2) % 12] = v[k2];
+    }
+  }
+};
+
 template <class T, int S> struct Bfly<T, 8, S> {
   static __device__ __forceinline__ void run(cx<T>* x) {
     const T h = T(0.70710678118654752440084436210484904);  // sqrt(2)/2

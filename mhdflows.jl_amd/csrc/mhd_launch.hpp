@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "mhd_kernels.hpp"
+#include "mhd_row.hpp"
 
 namespace mhd {
 
@@ -31,11 +32,13 @@ template <class T> inline int row_rows_per_block(int nx, int var = 0) {
   const int tx = m / row_plan_E(m, sizeof(T) == 8, var & 1);
   return 128 / tx;
 }
+// rows per workgroup of rowpair_kernel (RowPairShape::RPW)
+inline int rowpair_rows_per_block(int nx, int plan) { return 2 * (128 / (nx / rowpair_E(nx, plan))); }
 // most row blocks any variant needs (sizes the per-block partials)
 template <class T> inline int64_t row_blocks_max(int nx, int64_t rows) {
   int64_t b = 0;
   for (int v = 0; v < 2; ++v) {
-    const int64_t rpb = row_rows_per_block<T>(nx, v);
+    const int64_t rpb = std::min(row_rows_per_block<T>(nx, v), rowpair_rows_per_block(nx, v));
     b = std::max<int64_t>(b, (rows + rpb - 1) / rpb);
   }
   return b;
@@ -66,6 +69,9 @@ hipError_t launch_colpass(const ColArgs& a, int n, int dir, int S, const RunBuf<
 template <class T>
 hipError_t launch_xrow(const RowArgs& a, int kind, int nf, int var, const RunBuf<T>* runs, const cx<T>* twM,
                        const cx<T>* twh, hipStream_t s);
+template <class T>
+hipError_t launch_rowpair(const RowArgs& a, int kind, int plan, const RunBuf<T>* runs, const cx<T>* twx,
+                          hipStream_t s);
 template <class T>
 hipError_t launch_spectral(const SpecArgs& a, int phys, const RunBuf<T>* runs, hipStream_t s);
 template <class T>

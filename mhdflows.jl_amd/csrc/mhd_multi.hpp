@@ -14,6 +14,7 @@
 // persistent form, raised the column kernel from 84 to 166 VGPRs.)
 #pragma once
 #include "mhd_kernels.hpp"
+#include "mhd_row.hpp"
 
 namespace mhd {
 
@@ -66,8 +67,7 @@ struct MultiRow {
   int64_t start[MULTI_MAX + 1];
   RowArgs a[MULTI_MAX];
   const RunBuf<T>* runs[MULTI_MAX];
-  const cx<T>* twM[MULTI_MAX];
-  const cx<T>* twh[MULTI_MAX];
+  const cx<T>* twx[MULTI_MAX];
 };
 
 template <class T>
@@ -115,24 +115,30 @@ __global__ void __launch_bounds__(MULTI_THREADS) colpass_multi_kernel(MultiCol<T
 }
 
 // LDS bytes of a multi-size launch: column passes N*S + N complex values, rows the
-// RowShape exchange slots (plain index: M+1 per row) of the longest length in it
+// RowPairShape exchange slots of the largest in it
 template <class T> inline size_t multi_col_lds(int n) {
   return (size_t)(n * multi_col_strip(n) + n) * sizeof(cx<T>);
 }
 template <class T> inline size_t multi_row_lds(int nx, int pv) {
-  const int m = nx / 2;
-  const int tx = m / row_plan_E(m, sizeof(T) == 8, pv);
-  return (size_t)(128 / tx) * (m + 1) * sizeof(cx<T>);
+  int cx_slots = 0;
+#define MHD_MULTI_LDS(N_) \
+  if (nx == N_) cx_slots = pv ? RowPairShape<T, N_, 1>::LDS_CX : RowPairShape<T, N_, 0>::LDS_CX;
+  MHD_MULTI_LDS(32)
+  MHD_MULTI_LDS(48)
+  MHD_MULTI_LDS(64)
+  MHD_MULTI_LDS(96)
+  MHD_MULTI_LDS(128)
+#undef MHD_MULTI_LDS
+  return (size_t)cx_slots * sizeof(cx<T>);
 }
 
-// PV: the row plan (bit 0 of the row variant) of every group of the launch, so each run
-// computes with the plan its group's own launches use; the LDS index is the plain one
-// (the swizzled index, bit 1, changes no value).
-template <class T, int KIND, int NF, int PV>
+// PV: the row plan of every group of the launch, so each run computes with the plan its group's
+// own launches use.
+template <class T, int KIND, int PV>
 __global__ void __launch_bounds__(MULTI_THREADS) xrow_multi_kernel(MultiRow<T> m) {
   cx<T>* const xb = reinterpret_cast<cx<T>*>(multi_lds);  // dynamic: exchange slots of the longest row
   __shared__ T red[2 * 128];
-  __shared__ cx<T> stw[2 * 64 + 1];  // 2M+1 twiddles, M <= 64
+  __shared__ cx<T> stw[128];  // twiddles of rows of up to 128 points
   const int64_t it = blockIdx.x;
   if (it >= m.start[m.ngroups]) return;
   {
@@ -140,9 +146,9 @@ __global__ void __launch_bounds__(MULTI_THREADS) xrow_multi_kernel(MultiRow<T> m
     const int64_t item = it - m.start[g];
     const RowArgs& a = m.a[g];
     switch (m.nx[g]) {
-#define MHD_MULTI_ROW(N_)                                                                        \
-  case N_:                                                                                       \
-    xrow_item<T, N_, KIND, NF, PV>(a, item, m.runs[g], m.twM[g], m.twh[g], xb, red, stw);        \
+#define MHD_MULTI_ROW(N_)                                                              \
+  case N_:                                                                             \
+    rowpair_item<T, N_, KIND, PV>(a, item, m.runs[g], m.twx[g], xb, red, stw);         \
     break;
       MHD_MULTI_ROW(32)
       MHD_MULTI_ROW(48)
