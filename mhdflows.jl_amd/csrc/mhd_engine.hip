@@ -401,7 +401,7 @@ class Engine : public EngineBase {
   int rhs_rows_per_block(int var) const {
     return row_pairs() ? rowpair_rows_per_block(g.nx, var) : row_rows_per_block<T>(g.nx, var);
   }
-  int rhs_row_variant() const { return row_pairs() ? rowpair_plan(g.nx, phys) ^ (row_var & 1) : row_var; }
+  int rhs_row_variant() const { return row_pairs() ? rowpair_plan(g.nx, phys, sizeof(T) == 8) ^ (row_var & 1) : row_var; }
   RowArgs rhs_row_args(int var) const { return row_args_of(rhs_rows_per_block(var)); }
   // the other row launches: xrow_kernel, variant 0
   RowArgs row_args() const { return row_args_of(row_rows_per_block<T>(g.nx)); }

@@ -18,79 +18,152 @@
 // forward transforms from registers.  Twiddles are loaded once per work item and kept in
 // registers for all its transforms.
 //
+// A pass of radix R has B = N/R butterflies; thread t takes b = t, t + TX, ..., and where B is no
+// multiple of TX some threads sit a pass out: lengths 3 * 2^k then need few passes of radix 4 and
+// 8 in place of many of radix 2, and hold three or six values a thread instead of six or twelve.
+// The last inverse pass is always a full one, so the products are formed in its layout.
+//
 // Exchanges: LDS serves 128 B a cycle from 32 banks, i.e. G = 16 (Float32) or 8 (Float64) lanes of
 // a wave at a time, and slot s of a transform is in group s mod G.  Reads take consecutive
 // positions.  Writes of the pass with stride Ns and radix R take Ns consecutive positions out of
-// every Ns*R; C padding slots per G positions shift them apart (exch_pad).  Every exchange has
-// the C that its own write needs: none for Ns >= G.  Counted over all plans this leaves 1.0
-// cycles an access (1.5 in a few exchanges of the smallest lengths); one padding for all
-// exchanges of a plan had 28 % of the kernel's cycles in bank conflicts (256 points).  Indexes are
-// written as base + constant, which pad() keeps apart as their bits are disjoint (powers of two).
+// every Ns*R; padding slots shift them apart (Exchange): C per G positions where Ns*R is a power of
+// two, c per Ns*R positions otherwise, chosen for each exchange by its own writes.  One padding for
+// all exchanges of a plan had 28 % of the kernel's cycles in bank conflicts (256 points).  Slots are
+// written as base + constant.
 #pragma once
 #include "mhd_kernels.hpp"
 
 namespace mhd {
 
-// Row plans, by length and plan number: E values a thread and the radices, powers of two first.
+// Row plans, by length and plan number: E values a thread, the inverse radices, and the forward ones
+// (the same where they are powers of two, reversed otherwise).
+template <class L, bool REV> struct ForwardOrder { using type = L; };
+template <class L> struct ForwardOrder<L, true> { using type = typename RReverse<L>::type; };
 template <class T, int N, int P> struct RowPlan2;
 #define MHD_ROWPLAN2_B(N_, P_, E_, ...)              \
   template <class T> struct RowPlan2<T, N_, P_> {    \
     static constexpr int E = E_;                     \
     using R = Radices<__VA_ARGS__>;                  \
+    using F = typename ForwardOrder<R, (N_ % 3 == 0)>::type; \
   };
-// plan 0: eight values a thread (twelve for lengths with a factor 3)
+// plan 0: eight values a thread (three, six or twelve for lengths with a factor 3)
 MHD_ROWPLAN2_B(8, 0, 8, 8)
 MHD_ROWPLAN2_B(16, 0, 8, 8, 2)
-MHD_ROWPLAN2_B(24, 0, 12, 2, 12)
+MHD_ROWPLAN2_B(24, 0, 3, 8, 3)
 MHD_ROWPLAN2_B(32, 0, 8, 8, 4)
-MHD_ROWPLAN2_B(48, 0, 12, 4, 12)
+MHD_ROWPLAN2_B(48, 0, 6, 8, 6)
 MHD_ROWPLAN2_B(64, 0, 8, 8, 8)
-MHD_ROWPLAN2_B(96, 0, 12, 4, 2, 12)
+MHD_ROWPLAN2_B(96, 0, 3, 4, 8, 3)
 MHD_ROWPLAN2_B(128, 0, 8, 8, 8, 2)
-MHD_ROWPLAN2_B(192, 0, 12, 4, 4, 12)
+MHD_ROWPLAN2_B(192, 0, 6, 8, 4, 6)
 MHD_ROWPLAN2_B(256, 0, 8, 8, 8, 4)
-MHD_ROWPLAN2_B(384, 0, 12, 4, 4, 2, 12)
+MHD_ROWPLAN2_B(384, 0, 3, 4, 4, 8, 3)
 MHD_ROWPLAN2_B(512, 0, 8, 8, 8, 8)
 MHD_ROWPLAN2_B(768, 0, 12, 4, 4, 4, 12)
 MHD_ROWPLAN2_B(1024, 0, 8, 8, 8, 8, 2)
-// plan 1: four values a thread (six)
+// plan 1: four values a thread (three or six)
 MHD_ROWPLAN2_B(8, 1, 4, 4, 2)
 MHD_ROWPLAN2_B(16, 1, 4, 4, 4)
-MHD_ROWPLAN2_B(24, 1, 6, 2, 2, 6)
+MHD_ROWPLAN2_B(24, 1, 3, 4, 2, 3)
 MHD_ROWPLAN2_B(32, 1, 4, 4, 4, 2)
-MHD_ROWPLAN2_B(48, 1, 6, 2, 2, 2, 6)
+MHD_ROWPLAN2_B(48, 1, 3, 4, 4, 3)
 MHD_ROWPLAN2_B(64, 1, 4, 4, 4, 4)
-MHD_ROWPLAN2_B(96, 1, 6, 2, 2, 2, 2, 6)
+MHD_ROWPLAN2_B(96, 1, 3, 4, 4, 2, 3)
 MHD_ROWPLAN2_B(128, 1, 4, 4, 4, 4, 2)
-MHD_ROWPLAN2_B(192, 1, 6, 2, 2, 2, 2, 2, 6)
+MHD_ROWPLAN2_B(192, 1, 3, 4, 4, 4, 3)
 MHD_ROWPLAN2_B(256, 1, 4, 4, 4, 4, 4)
-MHD_ROWPLAN2_B(384, 1, 6, 2, 2, 2, 2, 2, 2, 6)
+MHD_ROWPLAN2_B(384, 1, 6, 8, 8, 6)
 MHD_ROWPLAN2_B(512, 1, 4, 4, 4, 4, 4, 2)
-MHD_ROWPLAN2_B(768, 1, 6, 2, 2, 2, 2, 2, 2, 2, 6)
+MHD_ROWPLAN2_B(768, 1, 6, 4, 4, 8, 6)
 MHD_ROWPLAN2_B(1024, 1, 16, 16, 16, 4)
-// The plan a row launch uses unless its variant asks for the other one.  Six fields (MHD) of four
-// values a thread fit 118 VGPRs (Float32: four waves a SIMD), of eight 221 (two); up to 512 points
-// the waves are worth more than the shorter sequence of passes (us a launch, plan 0 / plan 1:
-// Float32 64^3 17.3 / 14.0, 256^3 197 / 174, 512x256x128 201 / 194; Float64 256^3 414 / 341), for
-// longer rows the passes are (768x256x128 463 / 500, 1024x256x128 460 / 739).  Three fields (HD)
-// leave both plans their waves: four values only where launches are too small to fill the chip
-// (64^3 11.8 / 10.1, 192^3 47.5 / 55.2, 512x256x128 84 / 100).
-inline int rowpair_plan(int nx, int phys) { return nx <= (phys == PHYS_MHD ? 512 : 96) ? 1 : 0; }
+#undef MHD_ROWPLAN2_B
+// The plan a row launch uses unless its variant asks for the other one.  Six fields (MHD) of three
+// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 221 (two); up to 512
+// points the waves are worth more than the shorter sequence of passes (us a launch, plan 0 / plan 1:
+// Float32 64^3 17.3 / 14.0, 256^3 197 / 174, 512x256x128 201 / 194; Float64 256^3 414 / 341), at
+// 1024 the passes are (1024x256x128 460 / 739).  The lengths with a factor 3, where plan 1 was six
+// values in radix-2 passes and a last one of 6 (Float32 384x128x192 now 128, then 172; 768x256x192
+// 647, then 719 with twelve values; Float64 192^3 183, then 240; 384x128x192 291, then 315), plan
+// 0 / plan 1: Float32 48^3 15.8 / 13.4, 96^3 24.5 / 23.6, 192^3 89.8 / 82.0, 384x128x192 147 / 129;
+// Float64 192^3 209 / 183.  Three fields (HD) leave both plans their waves: fewer values only where
+// launches are too small to fill the chip (64^3 11.8 / 10.1, 192^3 43.1 / 48.3, 512x256x128
+// 84 / 100), at 384 points with their three passes (Float32 74 / 61, Float64 165 / 113) and at
+// 768 in Float64, where twelve values take the waves all the same (617 / 525, Float32 261 / 288).
+inline int rowpair_plan(int nx, int phys, bool f64) {
+  if (phys == PHYS_MHD) return nx < 1024 ? 1 : 0;
+  return nx <= 96 || nx == 384 || (nx == 768 && f64) ? 1 : 0;
+}
 // values a thread holds, for host-side launch shapes
 inline int rowpair_E(int nx, int plan) {
-  if (nx % 3 == 0) return plan ? 6 : 12;
-  if (nx == 1024) return plan ? 16 : 8;
-  return plan ? 4 : 8;
+  switch (nx) {
+#define MHD_ROW_E(N_) case N_: return plan ? RowPlan2<float, N_, 1>::E : RowPlan2<float, N_, 0>::E;
+    MHD_ROW_E(8) MHD_ROW_E(16) MHD_ROW_E(24) MHD_ROW_E(32) MHD_ROW_E(48) MHD_ROW_E(64) MHD_ROW_E(96)
+    MHD_ROW_E(128) MHD_ROW_E(192) MHD_ROW_E(256) MHD_ROW_E(384) MHD_ROW_E(512) MHD_ROW_E(768) MHD_ROW_E(1024)
+#undef MHD_ROW_E
+  }
+  return 8;
 }
-#undef MHD_ROWPLAN2_B
 
 template <class T> constexpr int lds_group() { return 128 / (int)sizeof(cx<T>); }
-template <class T> constexpr int exch_pad(int Ns, int R) {
-  const int G = lds_group<T>();
-  const int c = Ns >= G ? 0 : (Ns * R >= G ? (Ns == 1 ? 1 : G / R) : Ns);
-  return c > 4 ? 0 : c;
-}
 template <class T, int C> __host__ __device__ constexpr int pad(int pos) { return pos + C * (pos / lds_group<T>()); }
+
+// The exchange after the pass (Ns, R): slot of a written position base + r*Ns with
+// base = (b / Ns) * Ns*R + b % Ns, and of a read position b + r*B.
+template <class T, int Ns, int R> struct Exchange {
+  static constexpr int G = lds_group<T>(), NR = Ns * R;
+  static constexpr bool POW2 = (NR & (NR - 1)) == 0;
+  static constexpr int c2() {
+    const int c = Ns >= G ? 0 : (NR >= G ? (Ns == 1 ? 1 : G / R) : Ns);
+    return c > 4 ? 0 : c;
+  }
+  // lanes in the way of each other, summed over a wave's groups, with c padding slots per NR
+  static constexpr int conflicts(int c) {
+    int sum = 0;
+    for (int l0 = 0; l0 < 64; l0 += G) {
+      int worst = 0;
+      for (int s = 0; s < G; ++s) {
+        int n = 0;
+        for (int l = l0; l < l0 + G; ++l) n += ((l / Ns) * (NR + c) + l % Ns) % G == s ? 1 : 0;
+        worst = n > worst ? n : worst;
+      }
+      sum += worst;
+    }
+    return sum;
+  }
+  static constexpr int block_c() {
+    int best = 0;
+    for (int c = 1; c < G && c <= NR / 3; ++c) best = conflicts(c) < conflicts(best) ? c : best;
+    return best;
+  }
+  static constexpr int C = POW2 ? c2() : block_c();
+  static __device__ __forceinline__ int write_base(int b) {
+    if constexpr (POW2) return pad<T, C>((b / Ns) * NR + b % Ns);
+    else return (b / Ns) * (NR + C) + b % Ns;
+  }
+  static constexpr int write_step(int r) { return POW2 ? pad<T, C>(r * Ns) : r * Ns; }
+  // slots for N positions
+  static constexpr int slots(int N) { return POW2 ? pad<T, C>(N) : N + C * (N / NR); }
+  // read slot of b + r*B as base(b) + step(r*B); valid where separable<B>()
+  template <int B> static constexpr bool separable() { return POW2 ? B % G == 0 : B % NR == 0; }
+  static __device__ __forceinline__ int read_slot(int pos) { return POW2 ? pad<T, C>(pos) : pos + C * (pos / NR); }
+  static constexpr int read_step(int pos) { return POW2 ? pad<T, C>(pos) : pos + C * (pos / NR); }
+};
+// LDS slots a transform needs: the most of any exchange, and N/2 + 1 for the mirror exchange
+template <class T, int N, int Ns, class Rad> struct ExchangeSlots;
+template <class T, int N, int Ns, int R0> struct ExchangeSlots<T, N, Ns, Radices<R0>> {
+  static constexpr int value = N / 2 + 1;
+};
+template <class T, int N, int Ns, int R, int R2, int... Rest> struct ExchangeSlots<T, N, Ns, Radices<R, R2, Rest...>> {
+  static constexpr int a = Exchange<T, Ns, R>::slots(N), b = ExchangeSlots<T, N, Ns * R, Radices<R2, Rest...>>::value;
+  static constexpr int value = a > b ? a : b;
+};
+// values a thread holds during the passes: the most of any pass
+template <int N, int TX, class Rad> struct PassValues;
+template <int N, int TX> struct PassValues<N, TX, Radices<>> { static constexpr int value = 0; };
+template <int N, int TX, int R, int... Rest> struct PassValues<N, TX, Radices<R, Rest...>> {
+  static constexpr int a = (N / R + TX - 1) / TX * R, b = PassValues<N, TX, Radices<Rest...>>::value;
+  static constexpr int value = a > b ? a : b;
+};
 
 // Launch shape: 128 threads, LPW transforms at a time, each of two rows.
 template <class T, int NX, int PLAN> struct RowPairShape {
@@ -99,7 +172,9 @@ template <class T, int NX, int PLAN> struct RowPairShape {
   static constexpr int TX = NX / E;
   static constexpr int LPW = 128 / TX;
   static constexpr int RPW = 2 * LPW;                        // rows of a work item
-  static constexpr int SLOTS = pad<T, 4>(NX) + 2;            // + 2: transforms of one wave on other banks
+  static constexpr int EM = PassValues<NX, TX, typename P::R>::value;
+  static constexpr int SI = ExchangeSlots<T, NX, 1, typename P::R>::value, SF = ExchangeSlots<T, NX, 1, typename P::F>::value;
+  static constexpr int SLOTS = (SI > SF ? SI : SF) + 2;      // + 2: transforms of one wave on other banks
   static constexpr int LDS_CX = LPW * SLOTS;
   static_assert(128 % TX == 0, "a workgroup holds whole transforms");
 };
@@ -138,16 +213,16 @@ __device__ __forceinline__ T advective(int p, const T* v) {
 }
 
 // Twiddles of every pass but the first, in registers
-template <class T, int N, int E, int Ns, class Rad> struct RowTw;
-template <class T, int N, int E, int Ns> struct RowTw<T, N, E, Ns, Radices<>> {
+template <class T, int N, int TX, int Ns, class Rad> struct RowTw;
+template <class T, int N, int TX, int Ns> struct RowTw<T, N, TX, Ns, Radices<>> {
   __device__ __forceinline__ void load(int, const cx<T>*) {}
 };
-template <class T, int N, int E, int Ns, int R, int... Rest> struct RowTw<T, N, E, Ns, Radices<R, Rest...>> {
-  static constexpr int TX = N / E, NB = E / R;
+template <class T, int N, int TX, int Ns, int R, int... Rest> struct RowTw<T, N, TX, Ns, Radices<R, Rest...>> {
+  static constexpr int NB = (N / R + TX - 1) / TX;
   // butterflies t + i*TX whose index modulo Ns is the same share their twiddles
   static constexpr int NT = Ns == 1 ? 0 : (TX % Ns == 0 ? 1 : NB);
   cx<T> w[NT > 0 ? NT : 1][R > 1 ? R - 1 : 1];
-  RowTw<T, N, E, Ns * R, Radices<Rest...>> next;
+  RowTw<T, N, TX, Ns * R, Radices<Rest...>> next;
   __device__ __forceinline__ void load(int t, const cx<T>* tab) {
     if constexpr (Ns > 1) {
 #pragma unroll
@@ -161,54 +236,61 @@ template <class T, int N, int E, int Ns, int R, int... Rest> struct RowTw<T, N, 
   }
 };
 
-// One transform of direction S on x[j] = the value at position t + j*TX, in place.  row: the
-// transform's LDS slots.  A sync precedes every exchange write.
-template <class T, int N, int E, int S, bool WS, int Ns, class Rad> struct RowPass;
-template <class T, int N, int E, int S, bool WS, int Ns> struct RowPass<T, N, E, S, WS, Ns, Radices<>> {
+// One transform of direction S, in place: before a pass of radix R, x[i + r*NB] is the value at
+// position b + r*B, b = t + i*TX; after the last pass x[i + r*NB] is the value at b + r*B of that
+// pass.  row: the transform's LDS slots.  A sync precedes every exchange write.
+template <class T, int N, int TX, int S, bool WS, int Ns, class Rad> struct RowPass;
+template <class T, int N, int TX, int S, bool WS, int Ns> struct RowPass<T, N, TX, S, WS, Ns, Radices<>> {
   template <class Tw> static __device__ __forceinline__ void run(cx<T>*, int, cx<T>*, const Tw&) {}
 };
-template <class T, int N, int E, int S, bool WS, int Ns, int R, int... Rest>
-struct RowPass<T, N, E, S, WS, Ns, Radices<R, Rest...>> {
+template <class T, int N, int TX, int S, bool WS, int Ns, int R, int... Rest>
+struct RowPass<T, N, TX, S, WS, Ns, Radices<R, Rest...>> {
   template <class Tw>
   static __device__ __forceinline__ void run(cx<T>* x, int t, cx<T>* row, const Tw& tw) {
-    constexpr int TX = N / E, NB = E / R;
-    static_assert(E % R == 0, "radix must divide the values a thread holds");
+    constexpr int B = N / R, NB = (B + TX - 1) / TX;
     constexpr bool LAST = sizeof...(Rest) == 0;
-    constexpr int C = exch_pad<T>(Ns, R);
+    using X = Exchange<T, Ns, R>;
     if constexpr (!LAST) xsync<WS>();
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      cx<T> v[R];
+      const int b = t + i * TX;
+      if ((i + 1) * TX <= B || b < B) {
+        cx<T> v[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        v[r] = x[i + r * NB];
-        if constexpr (Ns > 1)
-          if (r > 0) v[r] = twmul<S>(v[r], tw.w[Tw::NT == 1 ? 0 : i][r > 0 ? r - 1 : 0]);
-      }
-      Bfly<T, R, S>::run(v);
-      if constexpr (LAST) {
-        // position b + r*Ns of butterfly b = t + i*TX, where Ns = N/R = NB*TX
+        for (int r = 0; r < R; ++r) {
+          v[r] = x[i + r * NB];
+          if constexpr (Ns > 1)
+            if (r > 0) v[r] = twmul<S>(v[r], tw.w[Tw::NT == 1 ? 0 : i][r > 0 ? r - 1 : 0]);
+        }
+        Bfly<T, R, S>::run(v);
+        if constexpr (LAST) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) x[i + r * NB] = v[r];
-      } else {
-        static_assert((Ns & (Ns - 1)) == 0 && (R & (R - 1)) == 0, "padded indexes add up for powers of two");
-        const int b = t + i * TX;
-        cx<T>* const d = row + pad<T, C>((b / Ns) * Ns * R + b % Ns);
+          for (int r = 0; r < R; ++r) x[i + r * NB] = v[r];
+        } else {
+          cx<T>* const d = row + X::write_base(b);
 #pragma unroll
-        for (int r = 0; r < R; ++r) d[pad<T, C>(r * Ns)] = v[r];
+          for (int r = 0; r < R; ++r) d[X::write_step(r)] = v[r];
+        }
       }
     }
     if constexpr (!LAST) {
       xsync<WS>();
-      if constexpr (TX % lds_group<T>() == 0) {
-        const cx<T>* const s = row + pad<T, C>(t);
+      constexpr int R2 = RFirst<Radices<Rest...>>::value, B2 = N / R2, NB2 = (B2 + TX - 1) / TX;
 #pragma unroll
-        for (int j = 0; j < E; ++j) x[j] = s[pad<T, C>(j * TX)];
-      } else {
+      for (int i = 0; i < NB2; ++i) {
+        const int b = t + i * TX;
+        if ((i + 1) * TX <= B2 || b < B2) {
+          if constexpr (X::template separable<B2>()) {
+            const cx<T>* const s = row + X::read_slot(b);
 #pragma unroll
-        for (int j = 0; j < E; ++j) x[j] = row[pad<T, C>(t + j * TX)];
+            for (int r = 0; r < R2; ++r) x[i + r * NB2] = s[X::read_step(r * B2)];
+          } else {
+#pragma unroll
+            for (int r = 0; r < R2; ++r) x[i + r * NB2] = row[X::read_slot(b + r * B2)];
+          }
+        }
       }
-      RowPass<T, N, E, S, WS, Ns * R, Radices<Rest...>>::run(x, t, row, tw.next);
+      RowPass<T, N, TX, S, WS, Ns * R, Radices<Rest...>>::run(x, t, row, tw.next);
     }
   }
 };
@@ -222,10 +304,17 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
   static_assert(KIND == ROW_MHD || KIND == ROW_HD, "the fused kinds");
   using SHP = RowPairShape<T, NX, PLAN>;
   using P = typename SHP::P;
-  using Rad = typename P::R;
-  constexpr int E = SHP::E, TX = SHP::TX, H = E / 2;
+  using Inv = typename P::R;
+  using Fwd = typename P::F;
+  constexpr int E = SHP::E, TX = SHP::TX, EM = SHP::EM;
   constexpr int NIN = KIND == ROW_MHD ? 6 : 3, NPROD = KIND == ROW_MHD ? NADV_MHD : NADV_HD;
   constexpr bool WS = TX <= 64;
+  // layouts of the half spectra: of the first inverse and the last forward pass
+  constexpr int R0 = RFirst<Inv>::value, B0 = NX / R0, N0 = (B0 + TX - 1) / TX, E0 = N0 * R0;
+  constexpr int RF = RLast<Fwd>::value, BF = NX / RF, NF_ = (BF + TX - 1) / TX;
+  constexpr int RL = RLast<Inv>::value;
+  static_assert(R0 % 2 == 0 && RF % 2 == 0, "a pass's upper half of positions mirrors the lower");
+  static_assert(NX / RL % TX == 0 && NX / RFirst<Fwd>::value % TX == 0 && E <= EM, "the products' layout is full");
 
   const int t = threadIdx.x;
   const int rw = t / TX, tr = t % TX;
@@ -243,13 +332,13 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
   __syncthreads();
   cx<T>* const xrow = xbuf + rw * SHP::SLOTS;
 
-  // The entries of the two half spectra of field f that position tr + j*TX takes: entry p for
-  // p < NX/2, the mirrored entry NX - p for p >= NX/2 (j >= E/2).  AHEAD fields are requested
-  // before the first transform starts, so the loads' latencies overlap.  Addresses are a uniform
-  // base (the item's first row of a field) plus a 32-bit offset and a constant.
-  constexpr int AHEAD = RowAhead<T, NIN, E>::value;
+  // The entries of the two half spectra of field f that position p = b + r*B0 takes: entry p for
+  // p < NX/2 (r < R0/2), the mirrored entry NX - p otherwise.  AHEAD fields are requested before
+  // the first transform starts, so the loads' latencies overlap.  Addresses are a uniform base (the
+  // item's first row of a field) plus a 32-bit offset and a constant.
+  constexpr int AHEAD = RowAhead<T, NIN, E0>::value;
   const int ncols = a.in_ncols;
-  cx<T> ra[NIN][E], rc[NIN][E];
+  cx<T> ra[NIN][E0], rc[NIN][E0];
   const int64_t ifs = field_stride(G, a.in_sel), irs = row_stride(G, a.in_sel);
   const int64_t ifirst = row_offset(G, a.in_sel, first);
   const gptr<const cx<T>> src = gmem<const cx<T>>(rb.buf[a.in_sel]) + (int64_t)a.in_f0 * ifs + ifirst;
@@ -259,40 +348,48 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
 #pragma unroll
     for (int f = f0; f < f1; ++f)
 #pragma unroll
-      for (int j = 0; j < E; ++j) ra[f][j] = rc[f][j] = cx<T>{T(0), T(0)};
+      for (int e = 0; e < E0; ++e) ra[f][e] = rc[f][e] = cx<T>{T(0), T(0)};
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      const int k = j < H ? tr + j * TX : (NX / 2 - tr) - (j - H) * TX;
-      if (k < ncols) {
+    for (int r = 0; r < R0; ++r)
 #pragma unroll
-        for (int f = f0; f < f1; ++f) {
-          const gptr<const cx<T>> pa = src + (int64_t)f * ifs, pc = pa + irs;
-          const uint32_t o = j < H ? iup + j * TX : idn - (j - H) * TX;
-          ra[f][j] = ldst<false, T>(pa + o);
-          rc[f][j] = ldst<false, T>(pc + o);
+      for (int i = 0; i < N0; ++i) {
+        const int b = tr + i * TX;
+        // entry up + b (r < R0/2) or down - b
+        const int up = r * B0, down = (R0 - r) * B0;
+        const int k = r < R0 / 2 ? up + b : down - b;
+        if (k < ncols && ((i + 1) * TX <= B0 || b < B0)) {
+          const uint32_t o = r < R0 / 2 ? iup + (up + i * TX) : idn - (NX / 2 - down + i * TX);
+#pragma unroll
+          for (int f = f0; f < f1; ++f) {
+            const gptr<const cx<T>> pa = src + (int64_t)f * ifs, pc = pa + irs;
+            ra[f][i + r * N0] = ldst<false, T>(pa + o);
+            rc[f][i + r * N0] = ldst<false, T>(pc + o);
+          }
         }
       }
-    }
   };
   request(0, AHEAD);
-  RowTw<T, NX, E, 1, Rad> tw;
-  tw.load(tr, stw);
 
-  // z[f][j].re, .im: field f at x = tr + j*TX of the two rows
+  // z[f][e].re, .im: field f of the two rows at x = tr + e*TX
   cx<T> z[NIN][E];
   const T scale = T(G.inv_n);
+  RowTw<T, NX, TX, 1, Inv> twi;
+  twi.load(tr, stw);
 #pragma unroll
   for (int f = 0; f < NIN; ++f) {
     if (f + AHEAD < NIN) request(f + AHEAD, f + AHEAD + 1);
+    cx<T> x[EM];
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      cx<T> A = ra[f][j], B = rc[f][j];
-      if ((j == 0 || j == H) && tr == 0) A.im = B.im = T(0);  // c2r ignores Im of the DC and Nyquist entries
-      z[f][j] = j < H ? cx<T>{A.re - B.im, A.im + B.re} : cx<T>{A.re + B.im, B.re - A.im};
+    for (int e = 0; e < E0; ++e) {
+      const int i = e % N0, r = e / N0;
+      cx<T> A = ra[f][e], B = rc[f][e];
+      // c2r ignores Im of the DC and Nyquist entries
+      if (i == 0 && (r == 0 || r == R0 / 2) && tr == 0) A.im = B.im = T(0);
+      x[e] = r < R0 / 2 ? cx<T>{A.re - B.im, A.im + B.re} : cx<T>{A.re + B.im, B.re - A.im};
     }
-    RowPass<T, NX, E, 1, WS, 1, Rad>::run(z[f], tr, xrow, tw);
+    RowPass<T, NX, TX, 1, WS, 1, Inv>::run(x, tr, xrow, twi);
 #pragma unroll
-    for (int j = 0; j < E; ++j) z[f][j] = z[f][j] * scale;
+    for (int e = 0; e < E; ++e) z[f][e] = x[e] * scale;
   }
 
   // A dealiased step's real fields would be overwritten by a later step of the same call before
@@ -350,12 +447,15 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
   const int64_t ofirst = row_offset(G, a.out_sel, first);
   const gptr<cx<T>> out = gmem(rb.buf[a.out_sel]) + (int64_t)a.out_f0 * ofs + ofirst;
   const uint32_t oup = (ok ? (uint32_t)(row_offset(G, a.out_sel, row0) - ofirst) : 0u) + tr;
+  RowTw<T, NX, TX, 1, Fwd> twf;
+  if constexpr (std::is_same<Inv, Fwd>::value) twf = twi;
+  else twf.load(tr, stw);
 #pragma unroll
   for (int i = 0; i < NPROD; ++i) {
     // the two diagonal products, which share their 22 entry, one after the other
     constexpr int ORDER[2][8] = {{0, 3, 1, 2, 4, 0, 0, 0}, {0, 6, 1, 2, 7, 3, 4, 5}};
     const int p = ORDER[KIND == ROW_MHD][i];
-    cx<T> w[E];
+    cx<T> w[EM];
 #pragma unroll
     for (int j = 0; j < E; ++j) {
       T v[NIN], u[NIN];
@@ -363,30 +463,37 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
       for (int f = 0; f < NIN; ++f) { v[f] = z[f][j].re; u[f] = z[f][j].im; }
       w[j] = cx<T>{advective<T, KIND>(p, v), advective<T, KIND>(p, u)};
     }
-    RowPass<T, NX, E, -1, WS, 1, Rad>::run(w, tr, xrow, tw);
-    // mirror exchange: the value at position q >= NX/2 goes to slot NX - q
+    RowPass<T, NX, TX, -1, WS, 1, Fwd>::run(w, tr, xrow, twf);
+    // mirror exchange: the value at position q = b + r*BF >= NX/2 goes to slot NX - q
     xsync<WS>();
-    {
-      cx<T>* const d = xrow + (NX / 2 - tr);
 #pragma unroll
-      for (int j = H; j < E; ++j) d[-(j - H) * TX] = w[j];
-    }
+    for (int r = RF / 2; r < RF; ++r)
+#pragma unroll
+      for (int ii = 0; ii < NF_; ++ii) {
+        const int b = tr + ii * TX;
+        if ((ii + 1) * TX <= BF || b < BF) xrow[(RF - r) * BF - b] = w[ii + r * NF_];
+      }
     xsync<WS>();
     // twice the product's half spectrum is stored (rhs_at halves it): no factor 1/2 here
     const gptr<cx<T>> da = out + (int64_t)p * ofs, dc = da + ors;
 #pragma unroll
-    for (int j = 0; j < H; ++j) {
-      const int k = tr + j * TX;
-      if (k < kend) {
-        cx<T> Zm = xrow[k];
-        if (j == 0 && tr == 0) Zm = w[0];  // entry 0 is its own mirror
-        stst<false, T>(da + (oup + j * TX), cx<T>{w[j].re + Zm.re, w[j].im - Zm.im});
-        stst<false, T>(dc + (oup + j * TX), cx<T>{w[j].im + Zm.im, Zm.re - w[j].re});
+    for (int r = 0; r < RF / 2; ++r)
+#pragma unroll
+      for (int ii = 0; ii < NF_; ++ii) {
+        const int b = tr + ii * TX, k = b + r * BF;
+        if (k < kend && ((ii + 1) * TX <= BF || b < BF)) {
+          const cx<T> Z = w[ii + r * NF_];
+          cx<T> Zm = xrow[k];
+          if (ii == 0 && r == 0 && tr == 0) Zm = Z;  // entry 0 is its own mirror
+          const uint32_t o = oup + (ii * TX + r * BF);
+          stst<false, T>(da + o, cx<T>{Z.re + Zm.re, Z.im - Zm.im});
+          stst<false, T>(dc + o, cx<T>{Z.im + Zm.im, Zm.re - Z.re});
+        }
       }
-    }
     if (NX / 2 < kend) {
       // the Nyquist entry is thread 0's value at position NX/2; zeros follow it to the line's end
-      const T nr = tr == 0 ? T(2) * w[H].re : T(0), ni = tr == 0 ? T(2) * w[H].im : T(0);
+      const cx<T> nq = w[RF / 2 * NF_];
+      const T nr = tr == 0 ? T(2) * nq.re : T(0), ni = tr == 0 ? T(2) * nq.im : T(0);
       for (int k = tr; k < kend - NX / 2; k += TX) {
         stst<false, T>(da + (oup + NX / 2 + (k - tr)), cx<T>{k == tr ? nr : T(0), T(0)});
         stst<false, T>(dc + (oup + NX / 2 + (k - tr)), cx<T>{k == tr ? ni : T(0), T(0)});

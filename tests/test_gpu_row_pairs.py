@@ -51,3 +51,21 @@ def test_small_magnetic_field_keeps_its_accuracy(n):
     N_gpu, _ = _calcN_gpu(p, o32.sol.copy())
     for f in (slice(0, 3), slice(3, 6)):
         assert rel_l2(N_gpu[f], N_ref[f]) < 2e-5
+
+
+# the long lengths with a factor 3, where some threads sit passes out; the Float32 bound of 128 points
+# grows with the largest wavenumber, which multiplies the products' rounding
+@pytest.mark.parametrize("nx", [192, 384, 768])
+@pytest.mark.parametrize("T", [np.float64, np.float32])
+@pytest.mark.parametrize("physics", ["MHD", "HD"])
+def test_rhs_long_rows_with_a_factor_3(nx, T, physics):
+    say("long rows", nx, T.__name__, physics)
+    mhd = physics == "MHD"
+    fields = _resample(ic.solenoidal_modes(6, k0=2.0, kmax=2.1, mhd=mhd), nx, 8, 24, mhd)
+    for var in (0, 1):
+        o, p = pair(nx, ny=8, nz=24, T=T, physics=physics, fields=fields)
+        M.variants(p, [-1, -1, -1, -1, var])
+        N_ref = np.zeros_like(o.sol)
+        N_gpu, _ = _calcN_gpu(p, o.sol.copy())
+        o_calcN(N_ref, o.sol.copy(), 0.0, o)
+        assert rel_l2(N_gpu, N_ref) < (1e-12 if T == np.float64 else 2e-5 * nx / 128), var
