@@ -83,6 +83,58 @@ int64_t run_bytes(const Geom& g, int phys, int prec) {
          (int64_t)nf * g.ny * g.nz * 2 * s + 4096;
 }
 
+// Time steps captured into HIP graphs: one of a single step and one of STEPS steps, each made when
+// a call first needs it.  Kernels within a graph follow each other without a gap, between two graphs
+// the device idles 8.3 us (traced at 64^3, where an LSRK54 step took 250 us); a call therefore
+// replays as many graphs of STEPS steps as it has room for.  Longer ones would save 1 us a step at
+// most and cost every call that makes them their instantiation.
+struct StepGraphs {
+  static constexpr int STEPS = 4;
+  hipGraph_t graph[2] = {nullptr, nullptr};  // of one step, of STEPS steps
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+
+  StepGraphs() = default;
+  StepGraphs(const StepGraphs&) = delete;
+  StepGraphs& operator=(const StepGraphs&) = delete;
+  ~StepGraphs() { drop(); }
+  void drop() {
+    for (int k = 0; k < 2; ++k) {
+      if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
+      if (graph[k]) (void)hipGraphDestroy(graph[k]);
+      exec[k] = nullptr;
+      graph[k] = nullptr;
+    }
+  }
+  template <class F> int capture(int k, hipStream_t s, F& step) {
+    if (exec[k]) return 0;
+    MHD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+    int rc = 0;
+    for (int i = 0; i < (k ? STEPS : 1) && rc == 0; ++i) rc = step();
+    hipGraph_t gr = nullptr;
+    const hipError_t e = hipStreamEndCapture(s, &gr);
+    if (rc) {
+      if (gr) (void)hipGraphDestroy(gr);
+      return rc;
+    }
+    if (e != hipSuccess) return fail(E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+    graph[k] = gr;
+    MHD_HIP(hipGraphInstantiate(&exec[k], gr, nullptr, nullptr, 0));
+    return 0;
+  }
+  // the graphs that a call of nsteps steps replays
+  template <class F> int ensure(int nsteps, hipStream_t s, F&& step) {
+    if (nsteps % STEPS) MHD_TRY(capture(0, s, step));
+    if (nsteps >= STEPS) MHD_TRY(capture(1, s, step));
+    return 0;
+  }
+  template <class F> int run(int nsteps, hipStream_t s, F&& step) {
+    MHD_TRY(ensure(nsteps, s, step));
+    for (; nsteps >= STEPS; nsteps -= STEPS) MHD_HIP(hipGraphLaunch(exec[1], s));
+    for (; nsteps > 0; --nsteps) MHD_HIP(hipGraphLaunch(exec[0], s));
+    return 0;
+  }
+};
+
 template <class T>
 class Engine : public EngineBase {
  public:
@@ -100,8 +152,7 @@ class Engine : public EngineBase {
   std::vector<RunClock> clk_init;
   const cx<T>*twy = nullptr, *twz = nullptr, *twM = nullptr, *twh = nullptr, *twx = nullptr;
   int64_t row_blocks = 0;
-  hipGraphExec_t gexec = nullptr;
-  hipGraph_t graph = nullptr;
+  StepGraphs graphs;
   bool use_graph = true;
   bool profiling = false;
   struct Ev {
@@ -123,8 +174,7 @@ class Engine : public EngineBase {
 
   ~Engine() override {
     if (st) hipStreamSynchronize(st);
-    if (gexec) hipGraphExecDestroy(gexec);
-    if (graph) hipGraphDestroy(graph);
+    graphs.drop();
     for (void* p : allocs) hipFree(p);
     for (void* p : force_tabs)
       if (p) hipFree(p);
@@ -328,7 +378,7 @@ class Engine : public EngineBase {
   };
 
   int colpass(const char* name, int axis, int dir, int src, int dst, int src_f0, int dst_f0, int nfields,
-              bool prune, bool hot = false, bool plane_out = false, bool prune_out = false) {
+              bool prune, bool hot = false, bool plane_out = false, bool prune_out = false, bool cfl = false) {
     const int n = axis == 1 ? g.ny : g.nz;
     const int S = (rec_ && rec_multi_) ? multi_col_strip(n) : col_strip<T>(n, hot ? col_var[col_class(axis, dir)] : 0);
     ColArgs a{};
@@ -368,6 +418,7 @@ class Engine : public EngineBase {
     a.gate = gate_;
     a.plane_out = plane_out ? 1 : 0;
     a.prune_out = prune_out ? 1 : 0;
+    a.cfl = cfl ? (phys == PHYS_MHD ? 2 : 1) : 0;
     const double cxb = sizeof(cx<T>);
     double bytes;
     if (prune_out && host_pruned_) {  // pruned step: kept columns (and pencils) only, kept outputs
@@ -675,11 +726,11 @@ class Engine : public EngineBase {
 
   // ---- one right-hand side evaluation ----------------------------------------
   // in_sel: stage input; prune: the stage input is dealiased; last: write vars + maxima.
-  int rhs(int in_sel, bool prune, SpecArgs sp, bool last) {
+  int rhs(int in_sel, bool prune, SpecArgs sp, bool last, bool first = false) {
     // a masked stage input has its kx = 0 plane copied aside by the z-pass, so the
     // spectral launch covers every mode at once (kx = 0 mirrors read from the copy)
     const bool fused_planes = prune && sp.mask_input && sp.self_sel < 0;
-    MHD_TRY(colpass("zpass_inv", 2, 1, in_sel, B_WORK, 0, 0, nf, prune, true, fused_planes));
+    MHD_TRY(colpass("zpass_inv", 2, 1, in_sel, B_WORK, 0, 0, nf, prune, true, fused_planes, false, first));
     // negative damping adds three products (f_i u_i) and its sum to the MHD row launch;
     // volume penalisation adds nf products chi/eta (v - V0) (u, and b for MHD) to every one
     const bool nd = nd_any && phys == PHYS_MHD && sp.add_force;
@@ -822,14 +873,13 @@ class Engine : public EngineBase {
   }
 
   int step_launches_gated() {
-    MHD_TRY(other("cfl", [this](hipStream_t s) { return launch_small<T>(SK_CFL, rbd, nr_, phys, 0, 0, s); }));
     if (stepper == STEP_RK4) {
       for (int s = 0; s < 4; ++s) {
         SpecArgs sp = spec_base();
         sp.mode = SP_RK4;
         sp.stage = s;
         sp.in_sel = s == 0 ? B_SOL : B_STIN;
-        MHD_TRY(rhs(sp.in_sel, true, sp, s == 3));
+        MHD_TRY(rhs(sp.in_sel, true, sp, s == 3, s == 0));
       }
     } else {
       static const double A[5] = {0.0, -567301805773.0 / 1357537059087.0, -2404267990393.0 / 2016746695238.0,
@@ -844,25 +894,9 @@ class Engine : public EngineBase {
         sp.in_sel = B_SOL;
         sp.ca = A[s];
         sp.cb = B[s];
-        MHD_TRY(rhs(B_SOL, true, sp, s == 4));
+        MHD_TRY(rhs(B_SOL, true, sp, s == 4, s == 0));
       }
     }
-    return 0;
-  }
-
-  int ensure_graph() {
-    if (gexec) return 0;
-    MHD_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    int rc = step_launches();
-    hipGraph_t gr = nullptr;
-    hipError_t e = hipStreamEndCapture(st, &gr);
-    if (rc) {
-      if (gr) hipGraphDestroy(gr);
-      return rc;
-    }
-    if (e != hipSuccess) return fail(E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-    graph = gr;
-    MHD_HIP(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
     return 0;
   }
 
@@ -870,9 +904,7 @@ class Engine : public EngineBase {
     if (nsteps < 0) return fail(E_INVALID, "nsteps must be >= 0");
     MHD_TRY(mark_prune(nsteps, st));  // the last of these steps (per run: or its target) is computed in full
     if (use_graph && !profiling) {
-      MHD_TRY(ensure_graph());
-      for (int i = 0; i < nsteps; ++i) MHD_HIP(hipGraphLaunch(gexec, st));
-      return 0;
+      return graphs.run(nsteps, st, [this] { return step_launches(); });
     }
     for (int i = 0; i < nsteps; ++i) MHD_TRY(step_launches());
     return 0;
@@ -1587,10 +1619,7 @@ class Engine : public EngineBase {
     return 0;
   }
   void drop_graph() {
-    if (gexec) (void)hipGraphExecDestroy(gexec);
-    if (graph) (void)hipGraphDestroy(graph);
-    gexec = nullptr;
-    graph = nullptr;
+    graphs.drop();
     ++graph_gen_;
   }
   int forcing_done() {
@@ -1816,7 +1845,7 @@ class Engine : public EngineBase {
     } ev;
     MHD_HIP(hipEventCreate(&ev.a));
     MHD_HIP(hipEventCreate(&ev.b));
-    if (use_graph) MHD_TRY(ensure_graph());
+    if (use_graph) MHD_TRY(graphs.ensure(nsteps, st, [this] { return step_launches(); }));
     MHD_HIP(hipStreamSynchronize(st));
     MHD_HIP(hipEventRecord(ev.a, st));
     MHD_TRY(step(nsteps));
@@ -1878,8 +1907,7 @@ class Engine : public EngineBase {
 // stepper): each group's step is recorded once, and the recordings are replayed position by
 // position -- one multi-size launch per hot launch (column passes, row kernel, spectral
 // update) for up to MULTI_MAX groups (row launches: groups of one row plan), the small
-// launches (CFL, maxima) per group -- on the first group's stream, captured as one HIP
-// graph per step.
+// launch (maxima) per group -- on the first group's stream, captured in HIP graphs.
 // ---------------------------------------------------------------------------
 template <class T>
 class FusedStep : public FusedBase {
@@ -1890,8 +1918,7 @@ class FusedStep : public FusedBase {
   std::vector<std::vector<Rec>> recm, recs;
   std::vector<uint64_t> gens;
   std::vector<hipEvent_t> evs;  // per group: its stream's pending work, then (index 0) our steps
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  StepGraphs graphs;
   bool use_graph = true;
   // per kernel class: one multi-size launch for all groups, or each group's own launch
   // (set by tune(); the spectral update is always multi-size)
@@ -1905,12 +1932,7 @@ class FusedStep : public FusedBase {
   }
   hipStream_t stream() const { return es[0]->st; }
 
-  void drop() {
-    if (gexec) (void)hipGraphExecDestroy(gexec);
-    if (graph) (void)hipGraphDestroy(graph);
-    gexec = nullptr;
-    graph = nullptr;
-  }
+  void drop() { graphs.drop(); }
 
   int init(const std::vector<EngineBase*>& groups) {
     for (EngineBase* b : groups) es.push_back(static_cast<Engine<T>*>(b));
@@ -1956,7 +1978,7 @@ class FusedStep : public FusedBase {
     const int ng_all = (int)es.size();
     const bool multi = type == Rec::SPEC || (type == Rec::COL && multi_col) || (type == Rec::ROW && multi_row);
     if (!multi) {
-      // the small launches (CFL, maxima) follow the row launches' shapes (block counts)
+      // the small launches (maxima) follow the row launches' shapes (block counts)
       const auto& R = (type == Rec::OTHER && multi_row) ? recm : recs;
       for (int k = 0; k < ng_all; ++k) {
         const hipError_t e = es[k]->launch_rec(R[k][i], s);
@@ -2022,24 +2044,6 @@ class FusedStep : public FusedBase {
     return 0;
   }
 
-  int ensure_graph() {
-    if (stale()) MHD_TRY(record());
-    if (gexec) return 0;
-    hipStream_t s = stream();
-    MHD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    const int rc = launch_step(s);
-    hipGraph_t gr = nullptr;
-    const hipError_t e = hipStreamEndCapture(s, &gr);
-    if (rc) {
-      if (gr) hipGraphDestroy(gr);
-      return rc;
-    }
-    if (e != hipSuccess) return fail(E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-    graph = gr;
-    MHD_HIP(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
-    return 0;
-  }
-
   // order the fused stream after the other groups' queued work
   int join_in(hipStream_t s) {
     for (size_t k = 1; k < es.size(); ++k) {
@@ -2060,11 +2064,10 @@ class FusedStep : public FusedBase {
     hipStream_t s = stream();
     MHD_TRY(join_in(s));
     for (Engine<T>* e : es) MHD_TRY(e->mark_prune(nsteps, s));
+    if (stale()) MHD_TRY(record());
     if (use_graph) {
-      MHD_TRY(ensure_graph());
-      for (int i = 0; i < nsteps; ++i) MHD_HIP(hipGraphLaunch(gexec, s));
+      MHD_TRY(graphs.run(nsteps, s, [&] { return launch_step(s); }));
     } else {
-      if (stale()) MHD_TRY(record());
       for (int i = 0; i < nsteps; ++i) MHD_TRY(launch_step(s));
     }
     return join_out(s);
@@ -2088,8 +2091,16 @@ class FusedStep : public FusedBase {
       if (r != hipSuccess) return fail(E_HIP, std::string("prune marks: ") + hipGetErrorString(r));
     }
     size_t first = 0, end = 0;  // [first, end): the first right-hand side's column and row launches
-    while (first < recm[0].size() && recm[0][first].type == Rec::OTHER) ++first;
-    end = first;
+    struct NoCfl {  // which choose no time step here
+      FusedStep* f;
+      explicit NoCfl(FusedStep* fs) : f(fs) { set(true); }
+      ~NoCfl() { set(false); }
+      void set(bool off) {
+        for (auto* recs : {&f->recm, &f->recs})
+          for (size_t k = 0; k < recs->size(); ++k)
+            (*recs)[k][0].ca.cfl = off ? 0 : (f->es[k]->phys == PHYS_MHD ? 2 : 1);
+      }
+    } no_cfl(this);
     while (end < recm[0].size() && recm[0][end].type != Rec::SPEC) ++end;
     struct Ev {
       hipEvent_t a = nullptr, b = nullptr;
