@@ -445,14 +445,24 @@ class Engine : public EngineBase {
     return timed(name, bytes, [&] { return launch_colpass<T>(a, n, dir, S, cur_rb(), tw, cs_); });
   }
 
-  // The fused row launch of a right-hand side: rowpair_kernel, or xrow_kernel for runs with a
-  // calcF! module or volume penalisation.  Variant row_var: of xrow_kernel as it is; for
-  // rowpair_kernel bit 0 picks the plan that rowpair_plan does not.
+  // The fused row launch of a right-hand side: rowpair_kernel or rowteam_kernel, or xrow_kernel for
+  // runs with a calcF! module or volume penalisation.  Variant row_var is xrow_kernel's own; for the
+  // others 0 is rowpair_choice, 1 the plan without teams (where that choice is teams) or the other
+  // plan, 2 and 3 are the teams ROW_TEAM and ROW_TEAM_HALF where the row length has them.
   bool row_pairs() const { return !active_module(); }
   int rhs_rows_per_block(int var) const {
     return row_pairs() ? rowpair_rows_per_block(g.nx, var) : row_rows_per_block<T>(g.nx, var);
   }
-  int rhs_row_variant() const { return row_pairs() ? rowpair_plan(g.nx, phys, sizeof(T) == 8) ^ (row_var & 1) : row_var; }
+  int rhs_row_variant() const { return rhs_row_variant(row_var); }
+  int rhs_row_variant(int v) const {
+    if (!row_pairs()) return v;
+    const bool f64 = sizeof(T) == 8;
+    const int plan = rowpair_plan(g.nx, phys, f64);
+    const int choice = rowpair_choice(g.nx, phys, f64, (int64_t)nr_ * g.ny * g.nz / 2);
+    int r = v >= 2 && rowteam_length(g.nx) ? v : choice;
+    if (v == 1) r = choice >= ROW_TEAM ? plan : plan ^ 1;
+    return rec_ && rec_multi_ && r >= ROW_TEAM ? 1 : r;  // multi-size launches have the plan without teams
+  }
   RowArgs rhs_row_args(int var) const { return row_args_of(rhs_rows_per_block(var)); }
   // the other row launches: xrow_kernel, variant 0
   RowArgs row_args() const { return row_args_of(row_rows_per_block<T>(g.nx)); }
@@ -661,8 +671,9 @@ class Engine : public EngineBase {
           if (dup) continue;
         } else {
           // xrow_kernel: bit 0 plan, bit 1 swizzled LDS; skip a plan equal to a lower variant's.
-          // rowpair_kernel: bit 0 plan
-          bool dup = row_pairs() && v > 1;
+          // Row pairs: skip what a lower variant launches
+          bool dup = false;
+          for (int u = 0; u < v; ++u) dup = dup || (row_pairs() && rhs_row_variant(u) == rhs_row_variant(v));
           for (int u = 0; u < v; ++u)
             if (!row_pairs() && (u >> 1) == (v >> 1) && row_rows_per_block<T>(g.nx, u) == row_rows_per_block<T>(g.nx, v)) dup = true;
           if (dup) continue;

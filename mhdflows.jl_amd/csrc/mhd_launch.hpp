@@ -32,13 +32,20 @@ template <class T> inline int row_rows_per_block(int nx, int var = 0) {
   const int tx = m / row_plan_E(m, sizeof(T) == 8, var & 1);
   return 128 / tx;
 }
-// rows per workgroup of rowpair_kernel (RowPairShape::RPW)
-inline int rowpair_rows_per_block(int nx, int plan) { return 2 * (128 / (nx / rowpair_E(nx, plan))); }
+// rows per workgroup of rowpair_kernel (RowPairShape::RPW) or rowteam_kernel (2 * RowTeamShape::LPT)
+inline int rowpair_rows_per_block(int nx, int plan) {
+  if (plan >= ROW_TEAM) return 2 * (64 / (nx / rowpair_E(nx, 1)));
+  return 2 * (128 / (nx / rowpair_E(nx, plan)));
+}
 // most row blocks any variant needs (sizes the per-block partials)
 template <class T> inline int64_t row_blocks_max(int nx, int64_t rows) {
   int64_t b = 0;
   for (int v = 0; v < 2; ++v) {
     const int64_t rpb = std::min(row_rows_per_block<T>(nx, v), rowpair_rows_per_block(nx, v));
+    b = std::max<int64_t>(b, (rows + rpb - 1) / rpb);
+  }
+  if (rowteam_length(nx)) {
+    const int64_t rpb = rowpair_rows_per_block(nx, ROW_TEAM);
     b = std::max<int64_t>(b, (rows + rpb - 1) / rpb);
   }
   return b;

@@ -104,6 +104,23 @@ inline int rowpair_E(int nx, int plan) {
   return 8;
 }
 
+// Row launches next to the two plans: rowteam_kernel (on plan 1) with a wave per product, or per two
+constexpr int ROW_TEAM = 2, ROW_TEAM_HALF = 3;
+inline bool rowteam_length(int nx) { return nx <= 256; }
+// The choice of a whole launch over `pairs` row pairs.  The waves of a plain launch each run 14 (HD:
+// 8) transforms one after the other; with less than about two of them a SIMD the launch takes as
+// long as one wave does, and teams shorten that.  us a launch, plain / a wave per product / per two,
+// by the waves of the plain launch: Float32 32^3 (64) 12.1 / 7.9 / 9.0, 64^3 (512) 15.9 / 12.2 / 13.2,
+// 128x64x64 (1024) 19.6 / 16.6 / 16.7, 96^3 (2304) 23.9 / 24.7 / 22.6, 128^3 (4096) 27.5 / 34.1 / 31.0;
+// Float64 64^3 18.8 / 15.2 / 15.9, 96^3 36.0 / 31.2 / 30.1, 128x96x64 (1536) 24.4 / 27.6 / 26.4.  Without
+// a magnetic field: Float32 32^3 9.2 / 7.3 / 7.8, 128x96x64 18.4 / 16.7 / 15.8, 128^3 20.1 / 24.2 / 20.9.
+inline int rowpair_choice(int nx, int phys, bool f64, int64_t pairs) {
+  const int64_t waves = pairs * (nx / rowpair_E(nx, 1)) / 64;
+  if (rowteam_length(nx) && waves < 768) return ROW_TEAM;
+  if (rowteam_length(nx) && waves < (f64 && nx % 3 ? 1280 : 2560)) return ROW_TEAM_HALF;
+  return rowpair_plan(nx, phys, f64);
+}
+
 template <class T> constexpr int lds_group() { return 128 / (int)sizeof(cx<T>); }
 template <class T, int C> __host__ __device__ constexpr int pad(int pos) { return pos + C * (pos / lds_group<T>()); }
 
@@ -177,6 +194,12 @@ template <class T, int NX, int PLAN> struct RowPairShape {
   static constexpr int SLOTS = (SI > SF ? SI : SF) + 2;      // + 2: transforms of one wave on other banks
   static constexpr int LDS_CX = LPW * SLOTS;
   static_assert(128 % TX == 0, "a workgroup holds whole transforms");
+  // layouts of the half spectra: of the first inverse and the last forward pass
+  static constexpr int R0 = RFirst<typename P::R>::value, B0 = NX / R0, N0 = (B0 + TX - 1) / TX, E0 = N0 * R0;
+  static constexpr int RF = RLast<typename P::F>::value, BF = NX / RF, NF = (BF + TX - 1) / TX;
+  static_assert(R0 % 2 == 0 && RF % 2 == 0, "a pass's upper half of positions mirrors the lower");
+  static_assert(NX / RLast<typename P::R>::value % TX == 0 && NX / RFirst<typename P::F>::value % TX == 0 && E <= EM,
+                "the products' layout is full");
 };
 
 // Fields requested ahead of the transforms: all of them where they fit the registers
@@ -188,28 +211,44 @@ template <class T, int NIN, int E> struct RowAhead {
 // The advective products of one point, u = v[0..2], b = v[3..5], in the order of NADV_MHD / NADV_HD:
 // T_ij = b_i b_j - u_i u_j and M_aj = u_a b_j - b_a u_j, or U_ij = u_i u_j, the diagonal entries
 // less the 22 entry.
+//
+// What is fused and what is rounded is spelled out, so that every launch that forms a product gives
+// the same bits.
+template <class T>
+__device__ __forceinline__ T diff2(T a, T b, T c, T d) { return fma(a, b, -(c * d)); }  // a b - c d
+template <class T>
+__device__ __forceinline__ T mul_rounded(T a, T b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
 template <class T, int KIND>
 __device__ __forceinline__ T advective(int p, const T* v) {
   if constexpr (KIND == ROW_MHD) {
     switch (p) {
-      case 0: return (v[3] * v[3] - v[0] * v[0]) - (v[5] * v[5] - v[2] * v[2]);
-      case 1: return v[3] * v[4] - v[0] * v[1];
-      case 2: return v[3] * v[5] - v[0] * v[2];
-      case 3: return v[0] * v[4] - v[3] * v[1];
-      case 4: return v[0] * v[5] - v[3] * v[2];
-      case 5: return v[1] * v[5] - v[4] * v[2];
-      case 6: return (v[4] * v[4] - v[1] * v[1]) - (v[5] * v[5] - v[2] * v[2]);
-      default: return v[4] * v[5] - v[1] * v[2];
+      case 0: return diff2(v[3], v[3], v[0], v[0]) - diff2(v[5], v[5], v[2], v[2]);
+      case 1: return diff2(v[3], v[4], v[0], v[1]);
+      case 2: return diff2(v[3], v[5], v[0], v[2]);
+      case 3: return diff2(v[0], v[4], v[3], v[1]);
+      case 4: return diff2(v[0], v[5], v[3], v[2]);
+      case 5: return diff2(v[1], v[5], v[4], v[2]);
+      case 6: return diff2(v[4], v[4], v[1], v[1]) - diff2(v[5], v[5], v[2], v[2]);
+      default: return diff2(v[4], v[5], v[1], v[2]);
     }
   } else {
     switch (p) {
-      case 0: return v[0] * v[0] - v[2] * v[2];
-      case 1: return v[0] * v[1];
-      case 2: return v[0] * v[2];
-      case 3: return v[1] * v[1] - v[2] * v[2];
-      default: return v[1] * v[2];
+      case 0: return diff2(v[0], v[0], v[2], v[2]);
+      case 1: return mul_rounded(v[0], v[1]);
+      case 2: return mul_rounded(v[0], v[2]);
+      case 3: return diff2(v[1], v[1], v[2], v[2]);
+      default: return mul_rounded(v[1], v[2]);
     }
   }
+}
+
+// a w, or a conj(w) for the inverse direction
+template <int S, class T> __device__ __forceinline__ cx<T> row_twmul(cx<T> a, cx<T> w) {
+  if (S < 0) return {diff2(a.re, w.re, a.im, w.im), fma(a.re, w.im, a.im * w.re)};
+  return {fma(a.re, w.re, a.im * w.im), diff2(a.im, w.re, a.re, w.im)};
 }
 
 // Twiddles of every pass but the first, in registers
@@ -260,7 +299,7 @@ struct RowPass<T, N, TX, S, WS, Ns, Radices<R, Rest...>> {
         for (int r = 0; r < R; ++r) {
           v[r] = x[i + r * NB];
           if constexpr (Ns > 1)
-            if (r > 0) v[r] = twmul<S>(v[r], tw.w[Tw::NT == 1 ? 0 : i][r > 0 ? r - 1 : 0]);
+            if (r > 0) v[r] = row_twmul<S>(v[r], tw.w[Tw::NT == 1 ? 0 : i][r > 0 ? r - 1 : 0]);
         }
         Bfly<T, R, S>::run(v);
         if constexpr (LAST) {
@@ -295,6 +334,57 @@ struct RowPass<T, N, TX, S, WS, Ns, Radices<R, Rest...>> {
   }
 };
 
+// The packed row of a pair of rows from their half-spectrum entries A, B of element e
+template <class T, int NX, class SHP>
+__device__ __forceinline__ cx<T> row_pack(cx<T> A, cx<T> B, int e, int tr) {
+  const int i = e % SHP::N0, r = e / SHP::N0;
+  // c2r ignores Im of the DC and Nyquist entries
+  if (i == 0 && (r == 0 || r == SHP::R0 / 2) && tr == 0) A.im = B.im = T(0);
+  return r < SHP::R0 / 2 ? cx<T>{A.re - B.im, A.im + B.re} : cx<T>{A.re + B.im, B.re - A.im};
+}
+
+// Store the half spectra of the two real rows whose packed transform is w (last forward pass's
+// layout): entries [0, kend) of each, at da + o and dc + o with o = oup + k - tr.
+template <class T, int NX, class SHP>
+__device__ __forceinline__ void row_store(const cx<T>* w, int tr, cx<T>* xrow, gptr<cx<T>> da, gptr<cx<T>> dc,
+                                          uint32_t oup, int kend) {
+  constexpr int TX = SHP::TX, RF = SHP::RF, BF = SHP::BF, NF = SHP::NF;
+  // mirror exchange: the value at position q = b + r*BF >= NX/2 goes to slot NX - q
+  xsync<(SHP::TX <= 64)>();
+#pragma unroll
+  for (int r = RF / 2; r < RF; ++r)
+#pragma unroll
+    for (int ii = 0; ii < NF; ++ii) {
+      const int b = tr + ii * TX;
+      if ((ii + 1) * TX <= BF || b < BF) xrow[(RF - r) * BF - b] = w[ii + r * NF];
+    }
+  xsync<(SHP::TX <= 64)>();
+  // twice the product's half spectrum is stored (rhs_at halves it): no factor 1/2 here
+#pragma unroll
+  for (int r = 0; r < RF / 2; ++r)
+#pragma unroll
+    for (int ii = 0; ii < NF; ++ii) {
+      const int b = tr + ii * TX, k = b + r * BF;
+      if (k < kend && ((ii + 1) * TX <= BF || b < BF)) {
+        const cx<T> Z = w[ii + r * NF];
+        cx<T> Zm = xrow[k];
+        if (ii == 0 && r == 0 && tr == 0) Zm = Z;  // entry 0 is its own mirror
+        const uint32_t o = oup + (ii * TX + r * BF);
+        stst<false, T>(da + o, cx<T>{Z.re + Zm.re, Z.im - Zm.im});
+        stst<false, T>(dc + o, cx<T>{Z.im + Zm.im, Zm.re - Z.re});
+      }
+    }
+  if (NX / 2 < kend) {
+    // the Nyquist entry is thread 0's value at position NX/2; zeros follow it to the line's end
+    const cx<T> nq = w[RF / 2 * NF];
+    const T nr = tr == 0 ? T(2) * nq.re : T(0), ni = tr == 0 ? T(2) * nq.im : T(0);
+    for (int k = tr; k < kend - NX / 2; k += TX) {
+      stst<false, T>(da + (oup + NX / 2 + (k - tr)), cx<T>{k == tr ? nr : T(0), T(0)});
+      stst<false, T>(dc + (oup + NX / 2 + (k - tr)), cx<T>{k == tr ? ni : T(0), T(0)});
+    }
+  }
+}
+
 // One work item (RPW rows of one run), run by a 128-thread workgroup.  xbuf holds
 // RowPairShape::LDS_CX exchange slots, red 2*128 values and stw NX twiddles.  Every early return
 // is taken by the whole workgroup.
@@ -309,12 +399,7 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
   constexpr int E = SHP::E, TX = SHP::TX, EM = SHP::EM;
   constexpr int NIN = KIND == ROW_MHD ? 6 : 3, NPROD = KIND == ROW_MHD ? NADV_MHD : NADV_HD;
   constexpr bool WS = TX <= 64;
-  // layouts of the half spectra: of the first inverse and the last forward pass
-  constexpr int R0 = RFirst<Inv>::value, B0 = NX / R0, N0 = (B0 + TX - 1) / TX, E0 = N0 * R0;
-  constexpr int RF = RLast<Fwd>::value, BF = NX / RF, NF_ = (BF + TX - 1) / TX;
-  constexpr int RL = RLast<Inv>::value;
-  static_assert(R0 % 2 == 0 && RF % 2 == 0, "a pass's upper half of positions mirrors the lower");
-  static_assert(NX / RL % TX == 0 && NX / RFirst<Fwd>::value % TX == 0 && E <= EM, "the products' layout is full");
+  constexpr int R0 = SHP::R0, B0 = SHP::B0, N0 = SHP::N0, E0 = SHP::E0;
 
   const int t = threadIdx.x;
   const int rw = t / TX, tr = t % TX;
@@ -380,13 +465,7 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
     if (f + AHEAD < NIN) request(f + AHEAD, f + AHEAD + 1);
     cx<T> x[EM];
 #pragma unroll
-    for (int e = 0; e < E0; ++e) {
-      const int i = e % N0, r = e / N0;
-      cx<T> A = ra[f][e], B = rc[f][e];
-      // c2r ignores Im of the DC and Nyquist entries
-      if (i == 0 && (r == 0 || r == R0 / 2) && tr == 0) A.im = B.im = T(0);
-      x[e] = r < R0 / 2 ? cx<T>{A.re - B.im, A.im + B.re} : cx<T>{A.re + B.im, B.re - A.im};
-    }
+    for (int e = 0; e < E0; ++e) x[e] = row_pack<T, NX, SHP>(ra[f][e], rc[f][e], e, tr);
     RowPass<T, NX, TX, 1, WS, 1, Inv>::run(x, tr, xrow, twi);
 #pragma unroll
     for (int e = 0; e < E; ++e) z[f][e] = x[e] * scale;
@@ -464,41 +543,8 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
       w[j] = cx<T>{advective<T, KIND>(p, v), advective<T, KIND>(p, u)};
     }
     RowPass<T, NX, TX, -1, WS, 1, Fwd>::run(w, tr, xrow, twf);
-    // mirror exchange: the value at position q = b + r*BF >= NX/2 goes to slot NX - q
-    xsync<WS>();
-#pragma unroll
-    for (int r = RF / 2; r < RF; ++r)
-#pragma unroll
-      for (int ii = 0; ii < NF_; ++ii) {
-        const int b = tr + ii * TX;
-        if ((ii + 1) * TX <= BF || b < BF) xrow[(RF - r) * BF - b] = w[ii + r * NF_];
-      }
-    xsync<WS>();
-    // twice the product's half spectrum is stored (rhs_at halves it): no factor 1/2 here
-    const gptr<cx<T>> da = out + (int64_t)p * ofs, dc = da + ors;
-#pragma unroll
-    for (int r = 0; r < RF / 2; ++r)
-#pragma unroll
-      for (int ii = 0; ii < NF_; ++ii) {
-        const int b = tr + ii * TX, k = b + r * BF;
-        if (k < kend && ((ii + 1) * TX <= BF || b < BF)) {
-          const cx<T> Z = w[ii + r * NF_];
-          cx<T> Zm = xrow[k];
-          if (ii == 0 && r == 0 && tr == 0) Zm = Z;  // entry 0 is its own mirror
-          const uint32_t o = oup + (ii * TX + r * BF);
-          stst<false, T>(da + o, cx<T>{Z.re + Zm.re, Z.im - Zm.im});
-          stst<false, T>(dc + o, cx<T>{Z.im + Zm.im, Zm.re - Z.re});
-        }
-      }
-    if (NX / 2 < kend) {
-      // the Nyquist entry is thread 0's value at position NX/2; zeros follow it to the line's end
-      const cx<T> nq = w[RF / 2 * NF_];
-      const T nr = tr == 0 ? T(2) * nq.re : T(0), ni = tr == 0 ? T(2) * nq.im : T(0);
-      for (int k = tr; k < kend - NX / 2; k += TX) {
-        stst<false, T>(da + (oup + NX / 2 + (k - tr)), cx<T>{k == tr ? nr : T(0), T(0)});
-        stst<false, T>(dc + (oup + NX / 2 + (k - tr)), cx<T>{k == tr ? ni : T(0), T(0)});
-      }
-    }
+    const gptr<cx<T>> da = out + (int64_t)p * ofs;
+    row_store<T, NX, SHP>(w, tr, xrow, da, da + ors, oup, kend);
   }
 }
 
@@ -512,6 +558,196 @@ rowpair_kernel(RowArgs a, const RunBuf<T>* __restrict__ runs, const cx<T>* __res
   const int64_t item = xcd_item(blockIdx.x, (int64_t)gridDim.x);
   if (item >= a.blocks_per_run * a.nruns) return;
   rowpair_item<T, NX, KIND, PLAN>(a, item, runs, twx, xb, red, stw);
+}
+
+// ---------------------------------------------------------------------------
+// The same launch for grids too small to fill the chip: a row pair's transforms side by side.
+// ---------------------------------------------------------------------------
+// Bound by latency: rowpair_kernel's waves there are fewer than SIMDs, and each runs its transforms
+// one after the other.  Here a workgroup of NT waves takes 64 / TX row pairs; wave q transforms the
+// fields q, q + NT, ... of all of them, leaves the real values in LDS, and after one barrier forms,
+// transforms and stores the products q, q + NT, ...  Field and product numbers are a wave's, so
+// nothing diverges.  A product reads four (HD: two) fields back from LDS, which costs more LDS
+// traffic and address arithmetic than the registers of rowpair_kernel: full chips take that one.
+// The results are rowpair_kernel's with plan 1, bit for bit.
+template <class T, int NX, int KIND, int NT> struct RowTeamShape {
+  using SHP = RowPairShape<T, NX, 1>;
+  static constexpr int TX = SHP::TX;
+  static constexpr int LPT = 64 / TX;                        // row pairs of a work item
+  static constexpr int NIN = KIND == ROW_MHD ? 6 : 3;
+  static constexpr int THREADS = 64 * NT;
+  static constexpr int LDS_CX = NT * LPT * SHP::SLOTS + NIN * LPT * NX;
+  static_assert(TX <= 64, "a wave holds whole transforms");
+};
+
+// Fields i, j of advective product p of NADV_MHD / NADV_HD
+__device__ __forceinline__ void advective_fields(int kind, int p, int* i, int* j) {
+  if (kind == ROW_MHD) {
+    *i = p >= 5 ? 1 : 0;
+    *j = p == 1 || p == 3 ? 1 : 2;
+  } else {
+    *i = p >= 3 ? 1 : 0;
+    *j = p == 1 ? 1 : 2;
+  }
+}
+
+template <class T, int NX, int KIND, int NT>
+__global__ void __launch_bounds__(64 * NT)
+rowteam_kernel(RowArgs a, const RunBuf<T>* __restrict__ runs, const cx<T>* __restrict__ twx) {
+  using TS = RowTeamShape<T, NX, KIND, NT>;
+  using SHP = typename TS::SHP;
+  using Inv = typename SHP::P::R;
+  using Fwd = typename SHP::P::F;
+  constexpr int E = SHP::E, TX = SHP::TX, EM = SHP::EM, LPT = TS::LPT;
+  constexpr int R0 = SHP::R0, B0 = SHP::B0, N0 = SHP::N0, E0 = SHP::E0;
+  constexpr int NIN = TS::NIN, NPROD = KIND == ROW_MHD ? NADV_MHD : NADV_HD;
+  constexpr int NFT = (NIN + NT - 1) / NT;  // fields a wave transforms, at most
+  __shared__ cx<T> lds[TS::LDS_CX];
+  __shared__ T red[2 * NT];
+  __shared__ cx<T> stw[NX];
+  const int64_t item = xcd_item(blockIdx.x, (int64_t)gridDim.x);
+  if (item >= a.blocks_per_run * a.nruns) return;
+
+  const int t = threadIdx.x, team = __builtin_amdgcn_readfirstlane(t / 64);
+  const int lane = t % 64, rw = lane / TX, tr = lane % TX;
+  const Geom& G = a.g;
+  const int run = (int)(item / a.blocks_per_run);
+  const int64_t blk = a.blk0 + item % a.blocks_per_run;
+  // rows as in rowpair_item
+  const int64_t first = blk * (2 * LPT), row0 = first + 2 * rw;
+  const bool ok = row0 < a.rows;
+  const RunBuf<T>& rb = runs[run];
+  if (gated_off(a.gate, rb)) return;
+  const bool pruned = a.prune_out && step_pruned(rb);
+  cx<T>* const xrow = lds + (team * LPT + rw) * SHP::SLOTS;
+  cx<T>* const zs = lds + NT * LPT * SHP::SLOTS + rw * NX + tr;  // field f's values at zs[f * LPT * NX + e * TX]
+
+  const int ncols = a.in_ncols;
+  cx<T> ra[NFT][E0], rc[NFT][E0];
+  const int64_t ifs = field_stride(G, a.in_sel), irs = row_stride(G, a.in_sel);
+  const int64_t ifirst = row_offset(G, a.in_sel, first);
+  const gptr<const cx<T>> src = gmem<const cx<T>>(rb.buf[a.in_sel]) + (int64_t)a.in_f0 * ifs + ifirst;
+  const uint32_t ioff = ok ? (uint32_t)(row_offset(G, a.in_sel, row0) - ifirst) : 0u;
+  const uint32_t iup = ioff + tr, idn = ioff + (NX / 2 - tr);  // entries tr, NX/2 - tr of row0
+#pragma unroll
+  for (int q = 0; q < NFT; ++q) {
+    const int f = team + q * NT;
+    const gptr<const cx<T>> pa = src + (int64_t)f * ifs, pc = pa + irs;
+#pragma unroll
+    for (int r = 0; r < R0; ++r)
+#pragma unroll
+      for (int i = 0; i < N0; ++i) {
+        const int b = tr + i * TX, up = r * B0, down = (R0 - r) * B0;
+        const int k = r < R0 / 2 ? up + b : down - b;
+        cx<T> A{T(0), T(0)}, B{T(0), T(0)};
+        if (f < NIN && k < ncols && ((i + 1) * TX <= B0 || b < B0)) {
+          const uint32_t o = r < R0 / 2 ? iup + (up + i * TX) : idn - (NX / 2 - down + i * TX);
+          A = ldst<false, T>(pa + o);
+          B = ldst<false, T>(pc + o);
+        }
+        ra[q][i + r * N0] = A;
+        rc[q][i + r * N0] = B;
+      }
+  }
+  for (int i = t; i < NX; i += TS::THREADS) stw[i] = twx[i];
+  __syncthreads();
+
+  const T scale = T(G.inv_n);
+  const bool put_vars = a.write_vars && !pruned && ok;
+  T mu = T(0), mb = T(0);
+  {
+    RowTw<T, NX, TX, 1, Inv> tw;
+    tw.load(tr, stw);
+#pragma unroll
+    for (int q = 0; q < NFT; ++q) {
+      const int f = team + q * NT;
+      if (f >= NIN) break;
+      cx<T> x[EM];
+#pragma unroll
+      for (int e = 0; e < E0; ++e) x[e] = row_pack<T, NX, SHP>(ra[q][e], rc[q][e], e, tr);
+      RowPass<T, NX, TX, 1, true, 1, Inv>::run(x, tr, xrow, tw);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        x[e] = x[e] * scale;
+        zs[f * (LPT * NX) + e * TX] = x[e];
+      }
+      if (put_vars) {
+        const gptr<T> va = gmem(rb.vars) + (int64_t)(a.real_out_f0 + f) * G.nr + first * NX;
+        const uint32_t o = (uint32_t)(2 * rw * NX + tr);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          va[o + e * TX] = x[e].re;
+          va[o + NX + e * TX] = x[e].im;
+        }
+      }
+      if (a.want_max) {
+        T m = T(0);
+#pragma unroll
+        for (int e = 0; e < E; ++e) m = nanmax(nanmax(m, fabs(x[e].re)), fabs(x[e].im));
+        if (f < 3) mu = nanmax(mu, m);
+        else mb = nanmax(mb, m);
+      }
+    }
+  }
+  if (a.want_max) {
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+      mu = nanmax(mu, __shfl_xor(mu, s));
+      mb = nanmax(mb, __shfl_xor(mb, s));
+    }
+    if (lane == 0) {
+      red[2 * team] = mu * mu;
+      red[2 * team + 1] = mb * mb;
+    }
+  }
+  __syncthreads();
+  if (a.want_max && t == 0) {
+    T m0 = red[0], m1 = red[1];
+    for (int q = 1; q < NT; ++q) {
+      m0 = nanmax(m0, red[2 * q]);
+      m1 = nanmax(m1, red[2 * q + 1]);
+    }
+    const gptr<T> part = gmem(rb.partial);
+    part[2 * blk] = m0;
+    part[2 * blk + 1] = m1;
+  }
+
+  const bool dst_work = a.out_sel == B_WORK;
+  const int kfull = dst_work ? G.wrs : NX / 2 + 1;
+  const int kend = !ok ? 0 : (pruned ? (dst_work ? G.kx_keep_w : G.kx_keep) : kfull);
+  const int64_t ofs = field_stride(G, a.out_sel), ors = row_stride(G, a.out_sel);
+  const int64_t ofirst = row_offset(G, a.out_sel, first);
+  const gptr<cx<T>> out = gmem(rb.buf[a.out_sel]) + (int64_t)a.out_f0 * ofs + ofirst;
+  const uint32_t oup = (ok ? (uint32_t)(row_offset(G, a.out_sel, row0) - ofirst) : 0u) + tr;
+  RowTw<T, NX, TX, 1, Fwd> tw;
+  tw.load(tr, stw);
+  for (int p = team; p < NPROD; p += NT) {
+    int fi, fj;
+    advective_fields(KIND, p, &fi, &fj);
+    const cx<T>* const zi = zs + fi * (LPT * NX);
+    const cx<T>* const zj = zs + fj * (LPT * NX);
+    cx<T> w[EM];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const cx<T> ui = zi[e * TX], uj = zj[e * TX];
+      if constexpr (KIND == ROW_MHD) {
+        const cx<T> bi = zi[3 * LPT * NX + e * TX], bj = zj[3 * LPT * NX + e * TX];
+        if (p == 0 || p == 6)
+          w[e] = cx<T>{diff2(bi.re, bi.re, ui.re, ui.re) - diff2(bj.re, bj.re, uj.re, uj.re),
+                       diff2(bi.im, bi.im, ui.im, ui.im) - diff2(bj.im, bj.im, uj.im, uj.im)};
+        else if (p >= 3 && p <= 5)
+          w[e] = cx<T>{diff2(ui.re, bj.re, bi.re, uj.re), diff2(ui.im, bj.im, bi.im, uj.im)};
+        else
+          w[e] = cx<T>{diff2(bi.re, bj.re, ui.re, uj.re), diff2(bi.im, bj.im, ui.im, uj.im)};
+      } else {
+        if (p == 0 || p == 3) w[e] = cx<T>{diff2(ui.re, ui.re, uj.re, uj.re), diff2(ui.im, ui.im, uj.im, uj.im)};
+        else w[e] = cx<T>{mul_rounded(ui.re, uj.re), mul_rounded(ui.im, uj.im)};
+      }
+    }
+    RowPass<T, NX, TX, -1, true, 1, Fwd>::run(w, tr, xrow, tw);
+    const gptr<cx<T>> da = out + (int64_t)p * ofs;
+    row_store<T, NX, SHP>(w, tr, xrow, da, da + ors, oup, kend);
+  }
 }
 
 }  // namespace mhd
