@@ -652,11 +652,21 @@ __device__ __forceinline__ T ipow(T x, int n) {
   return r;
 }
 
+// store of one entry of the state, whole in either form
+template <bool NT, class T> __device__ __forceinline__ void sst(gptr<cx<T>> p, cx<T> x) {
+  if constexpr (NT) {
+    stst<true, T>(p, x);
+  } else {
+    typedef T v2 __attribute__((ext_vector_type(2), aligned(sizeof(cx<T>))));
+    *(gptr<v2>)p = v2{x.re, x.im};
+  }
+}
+
 // qp: the mode's offset in the products buffer (its planes may be padded).  MODS = 0: the
 // advective products of rowpair_item, which stores twice their spectra (a power of two, so the 1/2
 // here is exact) and leaves out the 22 entry.  MODS = 1 (runs with a calcF! module or volume
 // penalisation, and the per-direction updates): the products of xrow_item.
-template <class T, int PHYS, int MODS>
+template <class T, int PHYS, int MODS, bool NT = true>
 __device__ __forceinline__ void rhs_at(const Geom& G, const RunBuf<T>& rb, const SpecArgs& a,
                                        int64_t qp, const ModeK<T>& k, const cx<T>* sH, cx<T>* R) {
   const gptr<const cx<T>> __restrict__ P = gmem<const cx<T>>(rb.buf[a.prod_sel]);
@@ -666,7 +676,7 @@ __device__ __forceinline__ void rhs_at(const Geom& G, const RunBuf<T>& rb, const
     constexpr int NP = nadv(PHYS);
     cx<T> p[NP];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) p[i] = ldst<true, T>(P + (int64_t)i * pfs + qp) * T(0.5);
+    for (int i = 0; i < NP; ++i) p[i] = ldst<NT, T>(P + (int64_t)i * pfs + qp) * T(0.5);
     // D_j = sum_i i k_i T_ij ; N_u = D - k (k.D)/k^2  (UᵢUpdate!, MHDSolver.jl:63-83; HD: N_u =
     // -P(i k . (u u)), HDSolver.jl:58-74)
     constexpr int SG = PHYS == PHYS_MHD ? 1 : -1;
@@ -688,7 +698,7 @@ __device__ __forceinline__ void rhs_at(const Geom& G, const RunBuf<T>& rb, const
     constexpr int NP = PHYS == PHYS_MHD ? 9 : 6;
     cx<T> p[NP];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) p[i] = ldst<true, T>(P + (int64_t)i * pfs + qp);
+    for (int i = 0; i < NP; ++i) p[i] = ldst<NT, T>(P + (int64_t)i * pfs + qp);
     if constexpr (PHYS == PHYS_MHD) {
       // D_j = sum_i i k_i T_ij ; N_u = D - k (k.D)/k^2  (UᵢUpdate!, MHDSolver.jl:63-83)
       const cx<T> d0 = mul_si<1>(p[0] * k.kx + p[1] * k.ky + p[2] * k.kz);
@@ -820,8 +830,9 @@ __device__ __forceinline__ void a99_add(const RunBuf<T>& rb, int kx, const ModeK
 }
 
 // MODS = 1 adds the calcF! modules (their registers would otherwise cost the plain launch
-// occupancy: 61 -> 72 VGPRs for Float32 MHD)
-template <class T, int PHYS, int PLANES, int MODS>
+// occupancy: 61 -> 72 VGPRs for Float32 MHD).  NT: non-temporal loads and stores, or ones that leave
+// the state in the caches for the launches that follow (launch_spectral).
+template <class T, int PHYS, int PLANES, int MODS, bool NT = true>
 __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>* __restrict__ runs, uint32_t i,
                                               int m, int run) {
   constexpr int NF = PHYS == PHYS_MHD ? 6 : 3;
@@ -885,7 +896,7 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       s[j][f] = zero;
-      if (j < nmodes && kept[j] && a.self_sel < 0) s[j][f] = ldst<true, T>(in + (int64_t)f * G.nc + qs[j]);
+      if (j < nmodes && kept[j] && a.self_sel < 0) s[j][f] = ldst<NT, T>(in + (int64_t)f * G.nc + qs[j]);
     }
   }
   if constexpr (!plane) {
@@ -930,7 +941,7 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
     }
     cx<T> R[NF];
     const int64_t qp = ms[j] * plane_stride(G, a.prod_sel) + ls[j] * row_stride(G, a.prod_sel) + kx;
-    rhs_at<T, PHYS, MODS>(G, rb, a, qp, k, sH, R);
+    rhs_at<T, PHYS, MODS, NT>(G, rb, a, qp, k, sH, R);
     if (MODS && rb.vp) {
       // VP_UᵢUpdate! / VP_BᵢUpdate! (src/Solver/VPSolver.jl:21-56): N_a += -(delta_aj - k_j k_a k^-2) P_j
       // for the penalisation products P of u (and b), which follow the advective ones
@@ -946,7 +957,7 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
 #pragma unroll
           for (int j = 0; j < 3; ++j) {
             const T coef = T(c == j ? 1 : 0) - kv[j] * kak2;
-            const cx<T> P = ldst<true, T>(Pv + (int64_t)(NADV + 3 * g + j) * pfs + qp);
+            const cx<T> P = ldst<NT, T>(Pv + (int64_t)(NADV + 3 * g + j) * pfs + qp);
             R[3 * g + c] = R[3 * g + c] + cx<T>{-coef * P.re, -coef * P.im};
           }
         }
@@ -966,7 +977,7 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
       if (MODS && rb.fdense) {  // N97ForceDriving! (src/pgen/TaylorGreenDynamo.jl:12-16): N_u += fh
         const gptr<const cx<T>> fdn = gmem<const cx<T>>(rb.fdense);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) R[c] = R[c] + ldst<true, T>(fdn + (int64_t)c * G.nc + q);
+        for (int c = 0; c < 3; ++c) R[c] = R[c] + ldst<NT, T>(fdn + (int64_t)c * G.nc + q);
       }
       if (MODS && rb.ndf) {  // NDForceDriving! (src/pgen/NegativeDamping.jl:40): N_u += A R2C(f u), A Float64
         const double A = rb.clk->nd_amp;
@@ -974,7 +985,7 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
         const int64_t pfs = field_stride(G, a.prod_sel);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          const cx<T> F = ldst<true, T>(Pn + (int64_t)(9 + c) * pfs + qp);
+          const cx<T> F = ldst<NT, T>(Pn + (int64_t)(9 + c) * pfs + qp);
           R[c] = cx<T>{T((double)R[c].re + A * (double)F.re), T((double)R[c].im + A * (double)F.im)};
         }
       }
@@ -1005,19 +1016,19 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
         cx<T> base = zero;
         if (kept[j]) {
           if (a.stage == 0) base = s[j][f];
-          else base = ldst<true, T>(sol + o);
+          else base = ldst<NT, T>(sol + o);
         }
         if (a.stage == 0) {
-          stst<true, T>(acc + o, cx<T>{R[f].re / T(6), R[f].im / T(6)});
-          if (kept[j]) stst<true, T>(stin + o, base + R[f] * half);
+          sst<NT, T>(acc + o, cx<T>{R[f].re / T(6), R[f].im / T(6)});
+          if (kept[j]) sst<NT, T>(stin + o, base + R[f] * half);
         } else if (a.stage == 1 || a.stage == 2) {
-          const cx<T> ac = ldst<true, T>(acc + o);
-          stst<true, T>(acc + o, cx<T>{ac.re + R[f].re / T(3), ac.im + R[f].im / T(3)});
-          if (kept[j]) stst<true, T>(stin + o, base + R[f] * (a.stage == 1 ? half : dt));
+          const cx<T> ac = ldst<NT, T>(acc + o);
+          sst<NT, T>(acc + o, cx<T>{ac.re + R[f].re / T(3), ac.im + R[f].im / T(3)});
+          if (kept[j]) sst<NT, T>(stin + o, base + R[f] * (a.stage == 1 ? half : dt));
         } else {
-          const cx<T> ac = ldst<true, T>(acc + o);
+          const cx<T> ac = ldst<NT, T>(acc + o);
           const cx<T> tot{ac.re + R[f].re / T(6), ac.im + R[f].im / T(6)};
-          stst<true, T>(sol + o, base + tot * dt);
+          sst<NT, T>(sol + o, base + tot * dt);
         }
       }
     } else {
@@ -1027,19 +1038,19 @@ __device__ __forceinline__ void spectral_item(const SpecArgs& a, const RunBuf<T>
       for (int f = 0; f < NF; ++f) {
         const int64_t o = (int64_t)f * G.nc + q;
         cx<T> Sold = zero;
-        if (a.stage != 0) Sold = ldst<true, T>(acc + o);
+        if (a.stage != 0) Sold = ldst<NT, T>(acc + o);
         const cx<T> Snew = Sold * A + R[f] * dt;
-        stst<true, T>(acc + o, Snew);
-        stst<true, T>(sol + o, s[j][f] + Snew * B);
+        sst<NT, T>(acc + o, Snew);
+        sst<NT, T>(sol + o, s[j][f] + Snew * B);
       }
     }
   }
 }
 
-template <class T, int PHYS, int PLANES, int MODS>
+template <class T, int PHYS, int PLANES, int MODS, bool NT = true>
 __global__ void __launch_bounds__(256)
 spectral_kernel(SpecArgs a, const RunBuf<T>* __restrict__ runs) {
-  spectral_item<T, PHYS, PLANES, MODS>(a, runs, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, blockIdx.z);
+  spectral_item<T, PHYS, PLANES, MODS, NT>(a, runs, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // ---------------------------------------------------------------------------
