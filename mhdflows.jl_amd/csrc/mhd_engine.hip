@@ -239,6 +239,7 @@ class Engine : public EngineBase {
     twh = twiddles<T>(device, g.nx, 1, &err);
     if (err) return err;
     row_blocks = row_blocks_max<T>(g.nx, (int64_t)g.ny * g.nz);  // partial capacity for any row variant
+    for (int c = 0; c < 4; ++c) col_var[c] = default_strip(c == 0 || c == 3 ? g.nz : g.ny);
     apply_cached_tuning();
     rbh.resize(nr_);
     force_tabs.assign(nr_, nullptr);
@@ -323,6 +324,11 @@ class Engine : public EngineBase {
   int col_var[4] = {0, 0, 0, 0};
   int row_var = 0;
 
+  // Strips of 128 B, or of 256 B for Float64 columns of 128 and 192 entries: twice the bytes a row of
+  // a strip for workgroups that still leave three or four a CU.  RK4 steps, ms, 128 B / 256 B: 96^3 0.426 /
+  // 0.443, 128^3 0.778 / 0.762, 192^3 2.586 / 2.492 (without a magnetic field 1.306 / 1.248), 256^3
+  // 5.74 / 5.77, 128x384x384 7.04 / 7.85.
+  static int default_strip(int n) { return sizeof(T) == 8 && n >= 128 && n < 256 ? 2 : 0; }
   static int col_class(int axis, int dir) { return dir > 0 ? (axis == 2 ? 0 : 1) : (axis == 1 ? 2 : 3); }
 
   int gate_ = 0;  // set while a time step is being launched
