@@ -285,9 +285,11 @@ int32_t mhd_autotune(mhd_handle* h, int32_t reps, char* report, int32_t report_l
 int32_t mhd_set_pipeline(mhd_handle* h, int32_t slabs);
 /* Set (v5 != NULL; negative entries keep the current value) and/or read (out5 != NULL)
  * the launch variants {zpass_inv, ypass_inv, ypass_fwd, zpass_fwd: strip width
- * 0 = 128 B, 1 = 64 B, 2 = 256 B, 3 = 512 B of kx per row; xrow_fused: bit 0 plan (Float32
- * powers of two: 0 = eight, 1 = four elements per thread), bit 1 XOR-swizzled LDS index
- * (0..3)}.  Results do not depend on the variant beyond floating-point rounding of the
+ * 0 = 128 B, 1 = 64 B, 2 = 256 B, 3 = 512 B of kx per row; xrow_fused: 0 = the default for the
+ * grid, 1 = the other row plan (or the plan alone where the default is a wave per product),
+ * 2, 3 = a wave per product, or per two products (rows of at most 256 points, the default
+ * elsewhere); for runs with a calcF! module: bit 0 plan (Float32 powers of two: 0 = eight,
+ * 1 = four elements per thread), bit 1 XOR-swizzled LDS index}.  Results do not depend on the variant beyond floating-point rounding of the
  * transform order. */
 int32_t mhd_set_variants(mhd_handle* h, const int32_t* v5, int32_t* out5);
 /* Time nsteps steps with HIP events on the handle's stream (whole-step wall time). */

@@ -14,8 +14,8 @@
 // magnitude (a seed magnetic field in a dynamo run).
 //
 // A transform of NX points belongs to TX = NX/E threads; thread t holds the positions t + j*TX
-// before the first and after the last pass, whatever the radices, so the products feed the
-// forward transforms from registers.  Twiddles are loaded once per work item and kept in
+// after the last inverse and before the first forward pass, whatever the radices, so the products
+// feed the forward transforms from registers.  Twiddles are loaded once per work item and kept in
 // registers for all its transforms.
 //
 // A pass of radix R has B = N/R butterflies; thread t takes b = t, t + TX, ..., and where B is no
