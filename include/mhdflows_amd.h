@@ -289,7 +289,8 @@ int32_t mhd_set_pipeline(mhd_handle* h, int32_t slabs);
  * grid, 1 = the other row plan (or the plan alone where the default is a wave per product),
  * 2, 3 = a wave per product, or per two products (rows of at most 256 points, the default
  * elsewhere); for runs with a calcF! module: bit 0 plan (Float32 powers of two: 0 = eight,
- * 1 = four elements per thread), bit 1 XOR-swizzled LDS index}.  Results do not depend on the variant beyond floating-point rounding of the
+ * 1 = four elements per thread), bit 1 the LDS index (plain or XOR-swizzled) that is not the
+ * default for the row length}.  Results do not depend on the variant beyond floating-point rounding of the
  * transform order. */
 int32_t mhd_set_variants(mhd_handle* h, const int32_t* v5, int32_t* out5);
 /* Time nsteps steps with HIP events on the handle's stream (whole-step wall time). */

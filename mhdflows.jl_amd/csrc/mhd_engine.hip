@@ -226,7 +226,8 @@ class Engine : public EngineBase {
     cs_ = st;
     {
       const int64_t rows = (int64_t)g.ny * g.nz;
-      pipe_ = (rows >= (int64_t)256 * 256 && rows <= (int64_t)512 * 512) ? 2 : 1;
+      pipe_ = rows < (int64_t)256 * 256 || rows > (int64_t)512 * 512 ? 1 : 2;
+      if (pipe_ == 2 && g.ny <= 256 && g.nz >= 256 && rows * g.nx >= (int64_t)192 * 256 * 256) pipe_ = 4;
     }
     MHD_HIP(hipStreamCreateWithFlags(&st2, hipStreamNonBlocking));  // default priority
     MHD_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
@@ -336,9 +337,13 @@ class Engine : public EngineBase {
   // pass act plane by plane, so over slabs of z-planes they run as pipe_ independent chains,
   // alternately on st and st2; the row kernel (VALU-bound) of one slab then overlaps the y passes
   // (memory-bound) of another.  slab_z0_/slab_z1_ bound the current slab (z1 < 0: none).
-  // Default: 2 slabs for planes of 256^2 to 512^2 rows (256^3 Float32 RK4: 321.5 -> 324.7
-  // steps/s; 4 slabs 322.9, 8 slabs 313.8); off below (launch-bound grids) and above (1024^3:
-  // 4.33 against 4.32 steps/s).
+  // Default: 2 slabs for grids of 256^2 to 512^2 rows, 4 where the planes have at most 256 rows and
+  // a quarter of the grid still fills the chip.  Float32 RK4 steps, ms, with 1 / 2 / 4 slabs:
+  // 256^3 2.924 / 2.906 / 2.828, 192x256x256 2.242 / 2.213 / 2.143, 128x256x512 3.193 / 3.154 / 3.062,
+  // 256x128x512 3.014 / 2.993 / 2.928 (256x256x384 alone lost: 4.432 / 4.438 / 4.462); smaller grids
+  // 96x256x256 1.166 / 1.152 / 1.219, 256x256x128 - / 1.394 / 1.402, larger planes 256x384x256
+  // - / 4.469 / 4.590, 512^3 25.06 / 24.99 / 25.01; without a magnetic field 256^3 - / 1.684 / 1.664,
+  // Float64 256^3 - / 5.512 / 5.441.  Off below (launch-bound grids) and above (1024^3: no gain).
   int pipe_ = 1;
   int slab_z0_ = 0, slab_z1_ = -1;
   // slab boundaries of the pipeline for row variant rvar (each slab starts on a whole row
@@ -452,8 +457,8 @@ class Engine : public EngineBase {
   }
 
   // The fused row launch of a right-hand side: rowpair_kernel or rowteam_kernel, or xrow_kernel for
-  // runs with a calcF! module or volume penalisation.  Variant row_var is xrow_kernel's own; for the
-  // others 0 is rowpair_choice, 1 the plan without teams (where that choice is teams) or the other
+  // runs with a calcF! module or volume penalisation.  Variant row_var: of xrow_kernel bit 0 its plan,
+  // bit 1 the other LDS index than its default; for the others 0 is rowpair_choice, 1 the plan without teams (where that choice is teams) or the other
   // plan, 2 and 3 are the teams ROW_TEAM and ROW_TEAM_HALF where the row length has them.
   bool row_pairs() const { return !active_module(); }
   int rhs_rows_per_block(int var) const {
@@ -461,7 +466,10 @@ class Engine : public EngineBase {
   }
   int rhs_row_variant() const { return rhs_row_variant(row_var); }
   int rhs_row_variant(int v) const {
-    if (!row_pairs()) return v;
+    // xrow_kernel's swizzled LDS index from 128 points (Float64: 64) up.  RK4 steps with a static force,
+    // ms, plain / swizzled: Float32 96^3 0.362 / 0.370, 128^3 0.522 / 0.508, 192^3 1.465 / 1.415, 256^3 3.67 /
+    // 3.39; Float64 48^3 0.273 / 0.276, 64^3 0.293 / 0.279, 128^3 0.932 / 0.897.  The bits do not depend on it.
+    if (!row_pairs()) return v ^ (g.nx >= (sizeof(T) == 8 ? 64 : 128) ? 2 : 0);
     const bool f64 = sizeof(T) == 8;
     const int plan = rowpair_plan(g.nx, phys, f64);
     const int choice = rowpair_choice(g.nx, phys, f64, (int64_t)nr_ * g.ny * g.nz / 2);
