@@ -287,7 +287,7 @@ int32_t mhd_set_pipeline(mhd_handle* h, int32_t slabs);
  * the launch variants {zpass_inv, ypass_inv, ypass_fwd, zpass_fwd: strip width
  * 0 = 128 B, 1 = 64 B, 2 = 256 B, 3 = 512 B of kx per row; xrow_fused: 0 = the default for the
  * grid, 1 = the other row plan (or the plan alone where the default is a wave per product),
- * 2, 3 = a wave per product, or per two products (rows of at most 256 points, the default
+ * 2, 3 = a wave per product, or three waves in all (rows of at most 256 points, the default
  * elsewhere); for runs with a calcF! module: bit 0 plan (Float32 powers of two: 0 = eight,
  * 1 = four elements per thread), bit 1 the LDS index (plain or XOR-swizzled) that is not the
  * default for the row length}.  Results do not depend on the variant beyond floating-point rounding of the

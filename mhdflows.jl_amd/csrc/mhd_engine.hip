@@ -76,7 +76,7 @@ double uniform01(uint64_t seed, uint64_t counter) {
 int64_t run_bytes(const Geom& g, int phys, int prec) {
   const int s = prec == 0 ? 4 : 8;
   const int nf = phys == PHYS_MHD ? 6 : 3;
-  const int np = work_fields(phys);
+  const int np = nprod(phys);
   const int64_t rows = (int64_t)g.ny * g.nz;
   const int64_t blocks = prec == 0 ? row_blocks_max<float>(g.nx, rows) : row_blocks_max<double>(g.nx, rows);
   return (int64_t)(3 * nf) * g.nc * 2 * s + (int64_t)np * g.wnc * 2 * s + (int64_t)nf * g.nr * s + 2 * blocks * s +
@@ -139,7 +139,7 @@ template <class T>
 class Engine : public EngineBase {
  public:
   Geom g{};
-  int phys = 0, nf = 0, np = 0 /* advective products without modules */, stepper = 0, nr_ = 0, dev = 0;
+  int phys = 0, nf = 0, np = 0, stepper = 0, nr_ = 0, dev = 0;
   hipStream_t st = nullptr;
   // Second stream and events of the slab pipeline (see rhs), and the stream the hot launches
   // go to (st, or st2 for odd slabs).
@@ -207,7 +207,7 @@ class Engine : public EngineBase {
     lens[2] = L[2];
     phys = ph;
     nf = ph == PHYS_MHD ? 6 : 3;
-    np = nadv(ph);
+    np = nprod(ph);
     stepper = stp;
     nr_ = (int)rp.size();
     dev = device;
@@ -248,7 +248,7 @@ class Engine : public EngineBase {
     ndf_bufs.assign(nr_, nullptr);
     ndpart_bufs.assign(nr_, nullptr);
     vp_bufs.assign(nr_, nullptr);
-    np_alloc = work_fields(phys);
+    np_alloc = np;
     for (int r = 0; r < nr_; ++r) {
       RunBuf<T>& b = rbh[r];
       std::memset(&b, 0, sizeof(b));
@@ -762,8 +762,7 @@ class Engine : public EngineBase {
     const bool vp = vp_any;
     const bool pairs = row_pairs();
     const int rvar = (nd || vp) ? 0 : rhs_row_variant();
-    const int nprod = pairs ? np : nprod_all(phys);
-    const int npf = nd ? nprod + 3 : (vp ? nprod + nf : nprod);
+    const int npf = nd ? np + 3 : (vp ? np + nf : np);
     RowArgs ra = rhs_row_args(rvar);
     ra.in_sel = B_WORK;
     ra.in_ncols = prune ? g.kx_keep : g.nkr;
@@ -844,7 +843,7 @@ class Engine : public EngineBase {
     const double c = sizeof(cx<T>) * (double)nr_;
     const double kept = (double)g.kx_keep * nkept_y(g) * nkept_z(g);
     const double all = (sp.gate && host_pruned_) ? kept : (double)g.nc;  // pruned step: kept modes only
-    double rd = ((row_pairs() ? np : nprod_all(phys)) + forcing_fields()) * all, wr = 0;
+    double rd = (np + forcing_fields()) * all, wr = 0;
     if (sp.mode == SP_RK4) {
       rd += nf * kept;                                  // stage input
       if (sp.stage > 0) rd += nf * kept + nf * all;     // base sol + acc
@@ -1222,8 +1221,8 @@ class Engine : public EngineBase {
     ra.out2_sel = B_STIN;
     ra.out2_f0 = 0;
     MHD_TRY(xrow("xrow_vars", ra, phys == PHYS_MHD ? ROW_VARS_MHD : ROW_VARS_HD, nf, 0));
-    MHD_TRY(colpass("ypass_fwd", 1, -1, B_WORK, B_WORK, 0, 0, nprod_all(phys), false));
-    MHD_TRY(colpass("zpass_fwd", 2, -1, B_WORK, B_WORK, 0, 0, nprod_all(phys), false));
+    MHD_TRY(colpass("ypass_fwd", 1, -1, B_WORK, B_WORK, 0, 0, np, false));
+    MHD_TRY(colpass("zpass_fwd", 2, -1, B_WORK, B_WORK, 0, 0, np, false));
     MHD_TRY(colpass("ypass_fwd", 1, -1, B_STIN, B_STIN, 0, 0, nf, false));
     MHD_TRY(colpass("zpass_fwd", 2, -1, B_STIN, B_STIN, 0, 0, nf, false));
     SpecArgs sp = spec_base();
@@ -1710,7 +1709,7 @@ class Engine : public EngineBase {
     }
     MHD_TRY(device_alloc(sizeof(double) * (size_t)row_blocks, &d));
     ndpart_bufs[run] = d;
-    if (phys == PHYS_MHD) MHD_TRY(grow_work(run, nprod_all(phys) + 3));  // room for the three f_i u_i products
+    if (phys == PHYS_MHD) MHD_TRY(grow_work(run, np + 3));  // room for the three f_i u_i products
     b.ndf = (const T*)ndf_bufs[run];
     b.ndpart = (double*)ndpart_bufs[run];
     b.nd_P = P;
@@ -1765,7 +1764,7 @@ class Engine : public EngineBase {
       if (phys == PHYS_MHD && B0 && B0[c])
         MHD_HIP(hipMemcpyAsync(base + (4 + c) * (size_t)g.nr, B0[c], fb, hipMemcpyHostToDevice, st));
     }
-    MHD_TRY(grow_work(run, nprod_all(phys) + nf));
+    MHD_TRY(grow_work(run, np + nf));
     b.vp = base;
     vp_any = true;
     drop_graph();

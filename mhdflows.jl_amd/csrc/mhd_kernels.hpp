@@ -164,8 +164,8 @@ colpass_kernel(ColArgs a, const RunBuf<T>* __restrict__ runs, const cx<T>* __res
 // row kernel: transforms along x of whole rows, with the real-space work fused
 // ---------------------------------------------------------------------------
 enum RowKind {
-  ROW_MHD = 0,        // 6 complex rows -> c2r -> 9 products (rowpair_item: 8) -> r2c
-  ROW_HD = 1,         // 3 complex rows -> c2r -> 6 products (rowpair_item: 5) -> r2c
+  ROW_MHD = 0,        // 6 complex rows -> c2r -> 9 products -> r2c
+  ROW_HD = 1,         // 3 complex rows -> c2r -> 6 products -> r2c
   ROW_C2R = 2,        // NF complex rows -> NF real rows
   ROW_R2C = 3,        // NF real rows -> NF complex rows
   ROW_VARS_MHD = 4,   // 6 real rows -> 9 products and the 6 inputs -> r2c (15 rows)
@@ -663,65 +663,37 @@ template <bool NT, class T> __device__ __forceinline__ void sst(gptr<cx<T>> p, c
 }
 
 // qp: the mode's offset in the products buffer (its planes may be padded).  MODS = 0: the
-// advective products of rowpair_item, which stores twice their spectra (a power of two, so the 1/2
-// here is exact) and leaves out the 22 entry.  MODS = 1 (runs with a calcF! module or volume
-// penalisation, and the per-direction updates): the products of xrow_item.
+// products of rowpair_item and rowteam_kernel, which store twice their spectra (a power of two, so
+// the 1/2 here is exact).  MODS = 1 (runs with a calcF! module or volume penalisation, and the
+// per-direction updates): the products of xrow_item.
 template <class T, int PHYS, int MODS, bool NT = true>
 __device__ __forceinline__ void rhs_at(const Geom& G, const RunBuf<T>& rb, const SpecArgs& a,
                                        int64_t qp, const ModeK<T>& k, const cx<T>* sH, cx<T>* R) {
+  constexpr int NP = PHYS == PHYS_MHD ? 9 : 6;
   const gptr<const cx<T>> __restrict__ P = gmem<const cx<T>>(rb.buf[a.prod_sel]);
   const int64_t pfs = field_stride(G, a.prod_sel);
+  cx<T> p[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    p[i] = ldst<NT, T>(P + (int64_t)i * pfs + qp);
+    if constexpr (MODS == 0) p[i] = p[i] * T(0.5);
+  }
   const cx<T> zero{T(0), T(0)};
-  if constexpr (MODS == 0) {
-    constexpr int NP = nadv(PHYS);
-    cx<T> p[NP];
-#pragma unroll
-    for (int i = 0; i < NP; ++i) p[i] = ldst<NT, T>(P + (int64_t)i * pfs + qp) * T(0.5);
-    // D_j = sum_i i k_i T_ij ; N_u = D - k (k.D)/k^2  (UᵢUpdate!, MHDSolver.jl:63-83; HD: N_u =
-    // -P(i k . (u u)), HDSolver.jl:58-74)
-    constexpr int SG = PHYS == PHYS_MHD ? 1 : -1;
-    constexpr int I11 = PHYS == PHYS_MHD ? 6 : 3, I12 = I11 + 1;
-    const cx<T> d0 = mul_si<SG>(p[0] * k.kx + p[1] * k.ky + p[2] * k.kz);
-    const cx<T> d1 = mul_si<SG>(p[1] * k.kx + p[I11] * k.ky + p[I12] * k.kz);
-    const cx<T> d2 = mul_si<SG>(p[2] * k.kx + p[I12] * k.ky);
-    const cx<T> kd = (d0 * k.kx + d1 * k.ky + d2 * k.kz) * k.invK;
-    R[0] = d0 - kd * k.kx;
-    R[1] = d1 - kd * k.ky;
-    R[2] = d2 - kd * k.kz;
-    if constexpr (PHYS == PHYS_MHD) {
-      // N_b_a = sum_{j != a} i k_j M_aj with M antisymmetric (BᵢUpdate!, MHDSolver.jl:147-158)
-      R[3] = mul_si<1>(p[3] * k.ky + p[4] * k.kz);
-      R[4] = mul_si<1>(p[5] * k.kz - p[3] * k.kx);
-      R[5] = mul_si<1>(zero - p[4] * k.kx - p[5] * k.ky);
-    }
-  } else {
-    constexpr int NP = PHYS == PHYS_MHD ? 9 : 6;
-    cx<T> p[NP];
-#pragma unroll
-    for (int i = 0; i < NP; ++i) p[i] = ldst<NT, T>(P + (int64_t)i * pfs + qp);
-    if constexpr (PHYS == PHYS_MHD) {
-      // D_j = sum_i i k_i T_ij ; N_u = D - k (k.D)/k^2  (UᵢUpdate!, MHDSolver.jl:63-83)
-      const cx<T> d0 = mul_si<1>(p[0] * k.kx + p[1] * k.ky + p[2] * k.kz);
-      const cx<T> d1 = mul_si<1>(p[1] * k.kx + p[3] * k.ky + p[4] * k.kz);
-      const cx<T> d2 = mul_si<1>(p[2] * k.kx + p[4] * k.ky + p[5] * k.kz);
-      const cx<T> kd = (d0 * k.kx + d1 * k.ky + d2 * k.kz) * k.invK;
-      R[0] = d0 - kd * k.kx;
-      R[1] = d1 - kd * k.ky;
-      R[2] = d2 - kd * k.kz;
-      // N_b_a = sum_{j != a} i k_j M_aj with M antisymmetric (BᵢUpdate!, MHDSolver.jl:147-158)
-      R[3] = mul_si<1>(p[6] * k.ky + p[7] * k.kz);
-      R[4] = mul_si<1>(p[8] * k.kz - p[6] * k.kx);
-      R[5] = mul_si<1>(zero - p[7] * k.kx - p[8] * k.ky);
-    } else {
-      // HD: N_u = -P(i k . (u u))  (HDSolver.jl:58-74)
-      const cx<T> d0 = mul_si<-1>(p[0] * k.kx + p[1] * k.ky + p[2] * k.kz);
-      const cx<T> d1 = mul_si<-1>(p[1] * k.kx + p[3] * k.ky + p[4] * k.kz);
-      const cx<T> d2 = mul_si<-1>(p[2] * k.kx + p[4] * k.ky + p[5] * k.kz);
-      const cx<T> kd = (d0 * k.kx + d1 * k.ky + d2 * k.kz) * k.invK;
-      R[0] = d0 - kd * k.kx;
-      R[1] = d1 - kd * k.ky;
-      R[2] = d2 - kd * k.kz;
-    }
+  // D_j = sum_i i k_i T_ij ; N_u = D - k (k.D)/k^2  (UᵢUpdate!, MHDSolver.jl:63-83; HD: N_u =
+  // -P(i k . (u u)), HDSolver.jl:58-74)
+  constexpr int SG = PHYS == PHYS_MHD ? 1 : -1;
+  const cx<T> d0 = mul_si<SG>(p[0] * k.kx + p[1] * k.ky + p[2] * k.kz);
+  const cx<T> d1 = mul_si<SG>(p[1] * k.kx + p[3] * k.ky + p[4] * k.kz);
+  const cx<T> d2 = mul_si<SG>(p[2] * k.kx + p[4] * k.ky + p[5] * k.kz);
+  const cx<T> kd = (d0 * k.kx + d1 * k.ky + d2 * k.kz) * k.invK;
+  R[0] = d0 - kd * k.kx;
+  R[1] = d1 - kd * k.ky;
+  R[2] = d2 - kd * k.kz;
+  if constexpr (PHYS == PHYS_MHD) {
+    // N_b_a = sum_{j != a} i k_j M_aj with M antisymmetric (BᵢUpdate!, MHDSolver.jl:147-158)
+    R[3] = mul_si<1>(p[6] * k.ky + p[7] * k.kz);
+    R[4] = mul_si<1>(p[8] * k.kz - p[6] * k.kx);
+    R[5] = mul_si<1>(zero - p[7] * k.kx - p[8] * k.ky);
   }
   constexpr int NF = PHYS == PHYS_MHD ? 6 : 3;
 #pragma unroll

@@ -78,17 +78,17 @@ MHD_ROWPLAN2_B(768, 1, 6, 4, 4, 8, 6)
 MHD_ROWPLAN2_B(1024, 1, 16, 16, 16, 4)
 #undef MHD_ROWPLAN2_B
 // The plan a row launch uses unless its variant asks for the other one.  Six fields (MHD) of three
-// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 221 (two); up to 512
-// points the waves are worth more than the shorter sequence of passes (us a launch, plan 0 / plan 1:
-// Float32 64^3 17.3 / 14.0, 256^3 197 / 174, 512x256x128 201 / 194; Float64 256^3 414 / 341), at
-// 1024 the passes are (1024x256x128 460 / 739).  The lengths with a factor 3, where plan 1 was six
-// values in radix-2 passes and a last one of 6 (Float32 384x128x192 now 128, then 172; 768x256x192
-// 647, then 719 with twelve values; Float64 192^3 183, then 240; 384x128x192 291, then 315), plan
-// 0 / plan 1: Float32 48^3 15.8 / 13.4, 96^3 24.5 / 23.6, 192^3 89.8 / 82.0, 384x128x192 147 / 129;
-// Float64 192^3 209 / 183.  Three fields (HD) leave both plans their waves: fewer values only where
-// launches are too small to fill the chip (64^3 11.8 / 10.1, 192^3 43.1 / 48.3, 512x256x128
-// 84 / 100), at 384 points with their three passes (Float32 74 / 61, Float64 165 / 113) and at
-// 768 in Float64, where twelve values take the waves all the same (617 / 525, Float32 261 / 288).
+// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 221 (two); up to 768
+// points the waves are worth more than the shorter sequence of passes, at 1024 the passes are.  us a
+// launch of a dealiased step, plan 0 / plan 1: Float32 192^3 95 / 90, 256^3 197 / 191, 384x128x192
+// 149 / 132, 1024x128x64 129 / 157 (against the rule 128^3 28.5 / 29.4, 512x256x128 203 / 214); Float64
+// 128^3 53 / 50, 192^3 206 / 188, 256x256x128 213 / 189.  Lengths with a factor 3 in six values of
+// radix-2 passes and a last one of 6 took 172 where 384x128x192 took 128 (768x256x192 719 with twelve
+// values / 647; Float64 192^3 240 / 183, 384x128x192 315 / 291).  Three fields (HD) leave both plans
+// their waves: fewer values only where launches are too small to fill the chip, at 384 points with
+// their three passes (Float32 81 / 68; Float64 165 / 113) and at 768 in Float64, where twelve values
+// take the waves all the same (617 / 525, Float32 261 / 288); otherwise plan 0 (256^3 96 / 99,
+// 512x256x128 84 / 100).
 inline int rowpair_plan(int nx, int phys, bool f64) {
   if (phys == PHYS_MHD) return nx < 1024 ? 1 : 0;
   return nx <= 96 || nx == 384 || (nx == 768 && f64) ? 1 : 0;
@@ -104,20 +104,25 @@ inline int rowpair_E(int nx, int plan) {
   return 8;
 }
 
-// Row launches next to the two plans: rowteam_kernel (on plan 1) with a wave per product, or per two
+// Row launches next to the two plans: rowteam_kernel (on plan 1) with a wave per product, or three
+// waves in all.  Three divide six fields and nine (HD: six) products without a rest; four and five
+// took 22.7 and 24.4 us at 96^3 for 21.7.
 constexpr int ROW_TEAM = 2, ROW_TEAM_HALF = 3;
 inline bool rowteam_length(int nx) { return nx <= 256; }
-// The choice of a whole launch over `pairs` row pairs.  The waves of a plain launch each run 14 (HD:
-// 8) transforms one after the other; with less than about two of them a SIMD the launch takes as
-// long as one wave does, and teams shorten that.  us a launch, plain / a wave per product / per two,
-// by the waves of the plain launch: Float32 32^3 (64) 12.1 / 7.9 / 9.0, 64^3 (512) 15.9 / 12.2 / 13.2,
-// 128x64x64 (1024) 19.6 / 16.6 / 16.7, 96^3 (2304) 23.9 / 24.7 / 22.6, 128^3 (4096) 27.5 / 34.1 / 31.0;
-// Float64 64^3 18.8 / 15.2 / 15.9, 96^3 36.0 / 31.2 / 30.1, 128x96x64 (1536) 24.4 / 27.6 / 26.4.  Without
-// a magnetic field: Float32 32^3 9.2 / 7.3 / 7.8, 128x96x64 18.4 / 16.7 / 15.8, 128^3 20.1 / 24.2 / 20.9.
+// The choice of a whole launch over `pairs` row pairs.  The waves of a plain launch each run 15 (HD:
+// 9) transforms one after the other; with less than about two of them a SIMD the launch takes as
+// long as one wave does, and teams shorten that.  us a launch, plain / a wave per product / three
+// waves, by the waves of the plain launch: Float32 32^3 (64) 12.0 / 8.0 / 9.0, 48^3 (288) 12.9 / 9.4 /
+// 10.2, 64^3 (512) 14.1 / 10.7 / 11.2, 128x64x64 (1024) 17.8 / 16.6 / 14.9, 256x64x64 (2048) 21.4 /
+// 26.9 / 22.0, 96^3 (2304) 23.1 / 29.7 / 21.7, 192x96x64 (3072) 25.6 / 37.5 / 26.5; Float64 32^3 13.8 /
+// 9.0 / 9.9, 48^3 14.8 / 12.8 / 11.6, 64^3 16.6 / 15.2 / 13.8, 96^3 37.1 / 47.6 / 31.1, 128x96x64 (1536)
+// 25.1 / 37.8 / 28.2.  Without a magnetic field:
+// Float32 32^3 9.5 / 7.0 / 7.4, 64^3 10.4 / 8.6 / 8.7, 128x96x64 16.0 / 14.1 / 13.3, 128^3 (4096)
+// 21.1 / 27.1 / 22.2; Float64 64^3 11.9 / 10.2 / 10.1, 128x96x64 20.2 / 22.5 / 18.9.
 inline int rowpair_choice(int nx, int phys, bool f64, int64_t pairs) {
   const int64_t waves = pairs * (nx / rowpair_E(nx, 1)) / 64;
-  if (rowteam_length(nx) && waves < 768) return ROW_TEAM;
-  if (rowteam_length(nx) && waves < (f64 && nx % 3 ? 1280 : 2560)) return ROW_TEAM_HALF;
+  if (rowteam_length(nx) && waves < (f64 && phys == PHYS_MHD ? 192 : 768)) return ROW_TEAM;
+  if (rowteam_length(nx) && waves < (nx % 3 && (f64 || phys == PHYS_MHD) ? 1280 : 2560)) return ROW_TEAM_HALF;
   return rowpair_plan(nx, phys, f64);
 }
 
@@ -208,9 +213,8 @@ template <class T, int NIN, int E> struct RowAhead {
   static constexpr int value = fit < NIN ? fit : NIN;
 };
 
-// The advective products of one point, u = v[0..2], b = v[3..5], in the order of NADV_MHD / NADV_HD:
-// T_ij = b_i b_j - u_i u_j and M_aj = u_a b_j - b_a u_j, or U_ij = u_i u_j, the diagonal entries
-// less the 22 entry.
+// The advective products of one point, u = v[0..2], b = v[3..5], in the order of nprod:
+// T_ij = b_i b_j - u_i u_j and M_ij = u_i b_j - b_i u_j, or U_ij = u_i u_j.
 //
 // What is fused and what is rounded is spelled out, so that every launch that forms a product gives
 // the same bits.
@@ -221,27 +225,17 @@ __device__ __forceinline__ T mul_rounded(T a, T b) {
 #pragma clang fp contract(off)
   return a * b;
 }
+// the indexes i, j of product p
+__host__ __device__ constexpr int advective_i(int p) { return p < 3 || p == 6 || p == 7 ? 0 : (p == 5 ? 2 : 1); }
+__host__ __device__ constexpr int advective_j(int p) { return p == 0 ? 0 : (p == 1 || p == 3 || p == 6 ? 1 : 2); }
 template <class T, int KIND>
 __device__ __forceinline__ T advective(int p, const T* v) {
+  const int i = advective_i(p), j = advective_j(p);
   if constexpr (KIND == ROW_MHD) {
-    switch (p) {
-      case 0: return diff2(v[3], v[3], v[0], v[0]) - diff2(v[5], v[5], v[2], v[2]);
-      case 1: return diff2(v[3], v[4], v[0], v[1]);
-      case 2: return diff2(v[3], v[5], v[0], v[2]);
-      case 3: return diff2(v[0], v[4], v[3], v[1]);
-      case 4: return diff2(v[0], v[5], v[3], v[2]);
-      case 5: return diff2(v[1], v[5], v[4], v[2]);
-      case 6: return diff2(v[4], v[4], v[1], v[1]) - diff2(v[5], v[5], v[2], v[2]);
-      default: return diff2(v[4], v[5], v[1], v[2]);
-    }
+    if (p < 6) return diff2(v[3 + i], v[3 + j], v[i], v[j]);
+    return diff2(v[i], v[3 + j], v[3 + i], v[j]);
   } else {
-    switch (p) {
-      case 0: return diff2(v[0], v[0], v[2], v[2]);
-      case 1: return mul_rounded(v[0], v[1]);
-      case 2: return mul_rounded(v[0], v[2]);
-      case 3: return diff2(v[1], v[1], v[2], v[2]);
-      default: return mul_rounded(v[1], v[2]);
-    }
+    return mul_rounded(v[i], v[j]);
   }
 }
 
@@ -397,7 +391,7 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
   using Inv = typename P::R;
   using Fwd = typename P::F;
   constexpr int E = SHP::E, TX = SHP::TX, EM = SHP::EM;
-  constexpr int NIN = KIND == ROW_MHD ? 6 : 3, NPROD = KIND == ROW_MHD ? NADV_MHD : NADV_HD;
+  constexpr int NIN = KIND == ROW_MHD ? 6 : 3, NPROD = KIND == ROW_MHD ? 9 : 6;
   constexpr bool WS = TX <= 64;
   constexpr int R0 = SHP::R0, B0 = SHP::B0, N0 = SHP::N0, E0 = SHP::E0;
 
@@ -530,10 +524,7 @@ __device__ __forceinline__ void rowpair_item(const RowArgs& a, int64_t item, con
   if constexpr (std::is_same<Inv, Fwd>::value) twf = twi;
   else twf.load(tr, stw);
 #pragma unroll
-  for (int i = 0; i < NPROD; ++i) {
-    // the two diagonal products, which share their 22 entry, one after the other
-    constexpr int ORDER[2][8] = {{0, 3, 1, 2, 4, 0, 0, 0}, {0, 6, 1, 2, 7, 3, 4, 5}};
-    const int p = ORDER[KIND == ROW_MHD][i];
+  for (int p = 0; p < NPROD; ++p) {
     cx<T> w[EM];
 #pragma unroll
     for (int j = 0; j < E; ++j) {
@@ -580,17 +571,6 @@ template <class T, int NX, int KIND, int NT> struct RowTeamShape {
   static_assert(TX <= 64, "a wave holds whole transforms");
 };
 
-// Fields i, j of advective product p of NADV_MHD / NADV_HD
-__device__ __forceinline__ void advective_fields(int kind, int p, int* i, int* j) {
-  if (kind == ROW_MHD) {
-    *i = p >= 5 ? 1 : 0;
-    *j = p == 1 || p == 3 ? 1 : 2;
-  } else {
-    *i = p >= 3 ? 1 : 0;
-    *j = p == 1 ? 1 : 2;
-  }
-}
-
 template <class T, int NX, int KIND, int NT>
 __global__ void __launch_bounds__(64 * NT)
 rowteam_kernel(RowArgs a, const RunBuf<T>* __restrict__ runs, const cx<T>* __restrict__ twx) {
@@ -600,7 +580,7 @@ rowteam_kernel(RowArgs a, const RunBuf<T>* __restrict__ runs, const cx<T>* __res
   using Fwd = typename SHP::P::F;
   constexpr int E = SHP::E, TX = SHP::TX, EM = SHP::EM, LPT = TS::LPT;
   constexpr int R0 = SHP::R0, B0 = SHP::B0, N0 = SHP::N0, E0 = SHP::E0;
-  constexpr int NIN = TS::NIN, NPROD = KIND == ROW_MHD ? NADV_MHD : NADV_HD;
+  constexpr int NIN = TS::NIN, NPROD = KIND == ROW_MHD ? 9 : 6;
   constexpr int NFT = (NIN + NT - 1) / NT;  // fields a wave transforms, at most
   __shared__ cx<T> lds[TS::LDS_CX];
   __shared__ T red[2 * NT];
@@ -722,26 +702,18 @@ rowteam_kernel(RowArgs a, const RunBuf<T>* __restrict__ runs, const cx<T>* __res
   RowTw<T, NX, TX, 1, Fwd> tw;
   tw.load(tr, stw);
   for (int p = team; p < NPROD; p += NT) {
-    int fi, fj;
-    advective_fields(KIND, p, &fi, &fj);
-    const cx<T>* const zi = zs + fi * (LPT * NX);
-    const cx<T>* const zj = zs + fj * (LPT * NX);
+    const cx<T>* const zi = zs + advective_i(p) * (LPT * NX);
+    const cx<T>* const zj = zs + advective_j(p) * (LPT * NX);
     cx<T> w[EM];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const cx<T> ui = zi[e * TX], uj = zj[e * TX];
       if constexpr (KIND == ROW_MHD) {
         const cx<T> bi = zi[3 * LPT * NX + e * TX], bj = zj[3 * LPT * NX + e * TX];
-        if (p == 0 || p == 6)
-          w[e] = cx<T>{diff2(bi.re, bi.re, ui.re, ui.re) - diff2(bj.re, bj.re, uj.re, uj.re),
-                       diff2(bi.im, bi.im, ui.im, ui.im) - diff2(bj.im, bj.im, uj.im, uj.im)};
-        else if (p >= 3 && p <= 5)
-          w[e] = cx<T>{diff2(ui.re, bj.re, bi.re, uj.re), diff2(ui.im, bj.im, bi.im, uj.im)};
-        else
-          w[e] = cx<T>{diff2(bi.re, bj.re, ui.re, uj.re), diff2(bi.im, bj.im, ui.im, uj.im)};
+        if (p < 6) w[e] = cx<T>{diff2(bi.re, bj.re, ui.re, uj.re), diff2(bi.im, bj.im, ui.im, uj.im)};
+        else w[e] = cx<T>{diff2(ui.re, bj.re, bi.re, uj.re), diff2(ui.im, bj.im, bi.im, uj.im)};
       } else {
-        if (p == 0 || p == 3) w[e] = cx<T>{diff2(ui.re, ui.re, uj.re, uj.re), diff2(ui.im, ui.im, uj.im, uj.im)};
-        else w[e] = cx<T>{mul_rounded(ui.re, uj.re), mul_rounded(ui.im, uj.im)};
+        w[e] = cx<T>{mul_rounded(ui.re, uj.re), mul_rounded(ui.im, uj.im)};
       }
     }
     RowPass<T, NX, TX, -1, true, 1, Fwd>::run(w, tr, xrow, tw);
