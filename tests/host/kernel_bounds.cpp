@@ -330,10 +330,10 @@ template <class T, int N, int PHYS> void spectral_forms(int stepper) {
 template <class T> void all() {
   spectral_forms<T, 64, PHYS_MHD>(SP_RK4);
   spectral_forms<T, 64, PHYS_MHD>(SP_LSRK54);
-  spectral_forms<T, 48, PHYS_HD>(SP_RK4);
+  spectral_forms<T, 24, PHYS_HD>(SP_RK4);
   steps<T, 16, 8, 24, PHYS_MHD>(SP_RK4);
-  steps<T, 64, 8, 8, PHYS_MHD>(SP_LSRK54);
-  steps<T, 96, 8, 8, PHYS_HD>(SP_RK4);
+  steps<T, 64, 8, 8, PHYS_MHD>(SP_RK4);
+  steps<T, 48, 8, 8, PHYS_HD>(SP_LSRK54);
 }
 }  // namespace
 
