@@ -471,8 +471,9 @@ class Engine : public EngineBase {
     // 3.39; Float64 48^3 0.273 / 0.276, 64^3 0.293 / 0.279, 128^3 0.932 / 0.897.  The bits do not depend on it.
     if (!row_pairs()) return v ^ (g.nx >= (sizeof(T) == 8 ? 64 : 128) ? 2 : 0);
     const bool f64 = sizeof(T) == 8;
-    const int plan = rowpair_plan(g.nx, phys, f64);
-    const int choice = rowpair_choice(g.nx, phys, f64, (int64_t)nr_ * g.ny * g.nz / 2);
+    const int64_t pairs = (int64_t)g.ny * g.nz / 2;
+    const int plan = rowpair_grid_plan(g.nx, phys, f64, pairs);
+    const int choice = rowpair_choice(g.nx, phys, f64, pairs, nr_);
     int r = v >= 2 && rowteam_length(g.nx) ? v : choice;
     if (v == 1) r = choice >= ROW_TEAM ? plan : plan ^ 1;
     return rec_ && rec_multi_ && r >= ROW_TEAM ? 1 : r;  // multi-size launches have the plan without teams

@@ -109,7 +109,7 @@ inline int rowpair_E(int nx, int plan) {
 // took 22.7 and 24.4 us at 96^3 for 21.7.
 constexpr int ROW_TEAM = 2, ROW_TEAM_HALF = 3;
 inline bool rowteam_length(int nx) { return nx <= 256; }
-// The choice of a whole launch over `pairs` row pairs.  The waves of a plain launch each run 15 (HD:
+// The team that a whole launch over `pairs` row pairs takes, 0 for none.  The waves of a plain launch each run 15 (HD:
 // 9) transforms one after the other; with less than about two of them a SIMD the launch takes as
 // long as one wave does, and teams shorten that.  us a launch, plain / a wave per product / three
 // waves, by the waves of the plain launch: Float32 32^3 (64) 12.0 / 8.0 / 9.0, 48^3 (288) 12.9 / 9.4 /
@@ -119,11 +119,21 @@ inline bool rowteam_length(int nx) { return nx <= 256; }
 // 25.1 / 37.8 / 28.2.  Without a magnetic field:
 // Float32 32^3 9.5 / 7.0 / 7.4, 64^3 10.4 / 8.6 / 8.7, 128x96x64 16.0 / 14.1 / 13.3, 128^3 (4096)
 // 21.1 / 27.1 / 22.2; Float64 64^3 11.9 / 10.2 / 10.1, 128x96x64 20.2 / 22.5 / 18.9.
-inline int rowpair_choice(int nx, int phys, bool f64, int64_t pairs) {
+inline int rowpair_team(int nx, int phys, bool f64, int64_t pairs) {
+  if (!rowteam_length(nx)) return 0;
   const int64_t waves = pairs * (nx / rowpair_E(nx, 1)) / 64;
-  if (rowteam_length(nx) && waves < (f64 && phys == PHYS_MHD ? 192 : 768)) return ROW_TEAM;
-  if (rowteam_length(nx) && waves < (nx % 3 && (f64 || phys == PHYS_MHD) ? 1280 : 2560)) return ROW_TEAM_HALF;
-  return rowpair_plan(nx, phys, f64);
+  if (waves < (f64 && phys == PHYS_MHD ? 384 : 768)) return ROW_TEAM;
+  return waves < (nx % 3 && (f64 || phys == PHYS_MHD) ? 1280 : 2560) ? ROW_TEAM_HALF : 0;
+}
+// The plan of a grid of `pairs` row pairs: plan 1 where one run is a team.  It does not depend on the
+// number of runs, so a run ends with the same bits alone and beside others.
+inline int rowpair_grid_plan(int nx, int phys, bool f64, int64_t pairs) {
+  return rowpair_team(nx, phys, f64, pairs) ? 1 : rowpair_plan(nx, phys, f64);
+}
+// The launch of `nruns` runs of such a grid: a team (then one run is one too) or the grid's plan.
+inline int rowpair_choice(int nx, int phys, bool f64, int64_t pairs, int nruns) {
+  const int team = rowpair_team(nx, phys, f64, pairs * nruns);
+  return team ? team : rowpair_grid_plan(nx, phys, f64, pairs);
 }
 
 template <class T> constexpr int lds_group() { return 128 / (int)sizeof(cx<T>); }
