@@ -274,7 +274,8 @@ int32_t mhd_restart(mhd_handle* h, const char* path, int32_t exact);
 /* ---- measurement -------------------------------------------------------------- */
 /* Autotuner: time every compiled variant of the hot launches (column-pass strip
  * widths, row-transform plans) with reps launches each, keep the fastest for this
- * grid and precision (for the process) and rebuild the captured step.  A text
+ * grid, precision and number of runs (for the process; the row transforms with and
+ * without a calcF! module apart) and rebuild the captured step.  A text
  * report of the timings is written to report (may be NULL). */
 int32_t mhd_autotune(mhd_handle* h, int32_t reps, char* report, int32_t report_len);
 /* Slab pipeline of each right-hand side: the y-inverse pass, the row kernel and the

@@ -320,10 +320,12 @@ class Engine : public EngineBase {
     return 0;
   }
 
-  // tuned variants: col_var[c] for the hot column passes c = zpass_inv, ypass_inv,
-  // ypass_fwd, zpass_fwd (strip width), row_var for the fused row kernel (plan)
+  // launch variants: col_var[c] for the hot column passes c = zpass_inv, ypass_inv, ypass_fwd,
+  // zpass_fwd (strip width), and one for each form of the fused row launch, whose numbers mean
+  // different things (rhs_row_variant): pair_var for row pairs and teams, xrow_var for xrow_kernel
   int col_var[4] = {0, 0, 0, 0};
-  int row_var = 0;
+  int pair_var = 0, xrow_var = 0;
+  int& row_var() { return row_pairs() ? pair_var : xrow_var; }
 
   // Strips of 128 B, or of 256 B for Float64 columns of 128 and 192 entries: twice the bytes a row of
   // a strip for workgroups that still leave three or four a CU.  RK4 steps, ms, 128 B / 256 B: 96^3 0.426 /
@@ -457,14 +459,15 @@ class Engine : public EngineBase {
   }
 
   // The fused row launch of a right-hand side: rowpair_kernel or rowteam_kernel, or xrow_kernel for
-  // runs with a calcF! module or volume penalisation.  Variant row_var: of xrow_kernel bit 0 its plan,
-  // bit 1 the other LDS index than its default; for the others 0 is rowpair_choice, 1 the plan without teams (where that choice is teams) or the other
-  // plan, 2 and 3 are the teams ROW_TEAM and ROW_TEAM_HALF where the row length has them.
+  // runs with a calcF! module or volume penalisation.  xrow_var: bit 0 its plan, bit 1 the other LDS
+  // index than its default.  pair_var: 0 is rowpair_choice, 1 the plan without teams (where that
+  // choice is teams) or the other plan, 2 and 3 are the teams ROW_TEAM and ROW_TEAM_HALF where the
+  // row length has them.
   bool row_pairs() const { return !active_module(); }
   int rhs_rows_per_block(int var) const {
     return row_pairs() ? rowpair_rows_per_block(g.nx, var) : row_rows_per_block<T>(g.nx, var);
   }
-  int rhs_row_variant() const { return rhs_row_variant(row_var); }
+  int rhs_row_variant() const { return rhs_row_variant(row_pairs() ? pair_var : xrow_var); }
   int rhs_row_variant(int v) const {
     // xrow_kernel's swizzled LDS index from 128 points (Float64: 64) up.  RK4 steps with a static force,
     // ms, plain / swizzled: Float32 96^3 0.362 / 0.370, 128^3 0.522 / 0.508, 192^3 1.465 / 1.415, 256^3 3.67 /
@@ -589,16 +592,24 @@ class Engine : public EngineBase {
     static std::map<std::string, std::vector<int>> c;
     return c;
   }
-  std::string tune_key() const {
+  // What a choice was measured for: the launches depend on the number of runs, and the row launch
+  // on whether a module acts.
+  std::string tune_key(bool pairs) const {
     return std::to_string(dev) + ":" + std::to_string(sizeof(T)) + ":" + std::to_string(g.nx) + "x" +
-           std::to_string(g.ny) + "x" + std::to_string(g.nz) + ":" + std::to_string(phys);
+           std::to_string(g.ny) + "x" + std::to_string(g.nz) + ":" + std::to_string(phys) + ":" + std::to_string(nr_) +
+           (pairs ? "" : ":module");
   }
+  // each row form's variant as tuned earlier in the process (a problem changes the form when its
+  // first module is set or its last one cleared)
   void apply_cached_tuning() {
     std::lock_guard<std::mutex> lk(g_tab_mu);
-    auto it = tune_cache().find(tune_key());
-    if (it == tune_cache().end()) return;
-    for (int c = 0; c < 4; ++c) col_var[c] = it->second[c];
-    row_var = it->second[4];
+    auto it = tune_cache().find(tune_key(true));
+    if (it != tune_cache().end()) {
+      for (int c = 0; c < 4; ++c) col_var[c] = it->second[c];
+      pair_var = it->second[4];
+    }
+    it = tune_cache().find(tune_key(false));
+    if (it != tune_cache().end()) xrow_var = it->second[4];
   }
 
   // time `reps` launches of one hot kernel with the given variant (work/stin only)
@@ -611,13 +622,13 @@ class Engine : public EngineBase {
       hipEvent_t a = nullptr, b = nullptr;
       ~Guard() {
         if (cls < 4) e->col_var[cls] = col;
-        else e->row_var = row;
+        else e->row_var() = row;
         if (a) hipEventDestroy(a);
         if (b) hipEventDestroy(b);
       }
-    } gd{this, cls, cls < 4 ? col_var[cls] : 0, row_var};
+    } gd{this, cls, cls < 4 ? col_var[cls] : 0, row_var()};
     if (cls < 4) col_var[cls] = var;
-    else row_var = var;
+    else row_var() = var;
     MHD_HIP(hipEventCreate(&gd.a));
     MHD_HIP(hipEventCreate(&gd.b));
     const hipEvent_t a = gd.a, b = gd.b;
@@ -710,10 +721,10 @@ class Engine : public EngineBase {
     gate_ = 0;
     MHD_HIP(launch_small<T>(SK_PRUNE, rbd, nr_, phys, 0, 0, st));
     for (int c = 0; c < 4; ++c) col_var[c] = best[c];
-    row_var = best[4];
+    row_var() = best[4];
     {
       std::lock_guard<std::mutex> lk(g_tab_mu);
-      tune_cache()[tune_key()] = best;
+      tune_cache()[tune_key(row_pairs())] = best;
     }
     drop_graph();
     return 0;
@@ -729,13 +740,13 @@ class Engine : public EngineBase {
         }
       if (v5[4] >= 0) {
         if (v5[4] > 3) return fail(E_INVALID, "row variant must be 0..3");
-        row_var = v5[4];
+        pair_var = xrow_var = v5[4];
       }
       drop_graph();
     }
     if (out5) {
       for (int c = 0; c < 4; ++c) out5[c] = col_var[c];
-      out5[4] = row_var;
+      out5[4] = row_var();
     }
     return 0;
   }
