@@ -294,6 +294,11 @@ int32_t mhd_set_pipeline(mhd_handle* h, int32_t slabs);
  * default for the row length}.  Results do not depend on the variant beyond floating-point rounding of the
  * transform order. */
 int32_t mhd_set_variants(mhd_handle* h, const int32_t* v5, int32_t* out5);
+/* Set (launch >= 0) and/or read (out != NULL) the row launch itself, for measurements and tests
+ * that must not depend on the choice for the grid: 0, 1 = the row plans, 2 = a wave per product,
+ * 3 = three waves (rows of at most 256 points).  mhd_set_variants with a row variant and
+ * mhd_autotune end it.  *out is -1 for runs with a calcF! module, which take none of these. */
+int32_t mhd_set_row_launch(mhd_handle* h, int32_t launch, int32_t* out);
 /* Time nsteps steps with HIP events on the handle's stream (whole-step wall time). */
 int32_t mhd_time_steps(mhd_handle* h, int32_t nsteps, double* ms_out);
 /* Run nsteps steps with an event pair around every kernel launch and report per

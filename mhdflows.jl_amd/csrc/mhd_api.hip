@@ -441,6 +441,10 @@ int32_t mhd_set_variants(mhd_handle* h, const int32_t* v5, int32_t* out5) {
   MHD_TRY(check_handle(h));
   return h->e->set_variants(v5, out5);
 }
+int32_t mhd_set_row_launch(mhd_handle* h, int32_t launch, int32_t* out) {
+  MHD_TRY(check_handle(h));
+  return h->e->set_row_launch(launch, out);
+}
 int32_t mhd_batch_autotune(mhd_batch* b, int32_t reps) {
   if (!b) return fail(E_INVALID, "batch is NULL");
   if (reps <= 0) return fail(E_INVALID, "reps must be > 0");

@@ -326,6 +326,7 @@ class Engine : public EngineBase {
   int col_var[4] = {0, 0, 0, 0};
   int pair_var = 0, xrow_var = 0;
   int& row_var() { return row_pairs() ? pair_var : xrow_var; }
+  int row_launch_ = -1;  // set_row_launch: the row-pair launch itself, whatever pair_var
 
   // Strips of 128 B, or of 256 B for Float64 columns of 128 and 192 entries: twice the bytes a row of
   // a strip for workgroups that still leave three or four a CU.  RK4 steps, ms, 128 B / 256 B: 96^3 0.426 /
@@ -467,7 +468,10 @@ class Engine : public EngineBase {
   int rhs_rows_per_block(int var) const {
     return row_pairs() ? rowpair_rows_per_block(g.nx, var) : row_rows_per_block<T>(g.nx, var);
   }
-  int rhs_row_variant() const { return rhs_row_variant(row_pairs() ? pair_var : xrow_var); }
+  int rhs_row_variant() const {
+    if (row_pairs() && row_launch_ >= 0) return row_launch_;
+    return rhs_row_variant(row_pairs() ? pair_var : xrow_var);
+  }
   int rhs_row_variant(int v) const {
     // xrow_kernel's swizzled LDS index from 128 points (Float64: 64) up.  RK4 steps with a static force,
     // ms, plain / swizzled: Float32 96^3 0.362 / 0.370, 128^3 0.522 / 0.508, 192^3 1.465 / 1.415, 256^3 3.67 /
@@ -677,6 +681,7 @@ class Engine : public EngineBase {
   // Uses work and stin as scratch (their contents are dead between steps).
   int autotune(int reps, std::string* report) {
     if (reps <= 0) reps = 5;
+    row_launch_ = -1;
     MHD_HIP(hipStreamSynchronize(st));
     const char* names[5] = {"zpass_inv", "ypass_inv", "ypass_fwd", "zpass_fwd", "xrow_fused"};
     std::vector<int> best(5, 0);
@@ -741,6 +746,7 @@ class Engine : public EngineBase {
       if (v5[4] >= 0) {
         if (v5[4] > 3) return fail(E_INVALID, "row variant must be 0..3");
         pair_var = xrow_var = v5[4];
+        row_launch_ = -1;
       }
       drop_graph();
     }
@@ -748,6 +754,18 @@ class Engine : public EngineBase {
       for (int c = 0; c < 4; ++c) out5[c] = col_var[c];
       out5[4] = row_var();
     }
+    return 0;
+  }
+
+  int set_row_launch(int launch, int* out) override {
+    if (launch >= 0) {
+      if (!row_pairs()) return fail(E_UNSUPPORTED, "a module's runs have no row-pair launch");
+      if (launch > ROW_TEAM_HALF || (launch >= ROW_TEAM && !rowteam_length(g.nx)))
+        return fail(E_INVALID, "row launch must be 0..3, and 2, 3 need rows of at most 256 points");
+      row_launch_ = launch;
+      drop_graph();
+    }
+    if (out) *out = row_pairs() ? rhs_row_variant() : -1;
     return 0;
   }
 

@@ -98,6 +98,7 @@ class EngineBase {
   virtual int start_run(int run, double dt, double cfl_coef, int64_t target) = 0;
   virtual int query() = 0;  // 1 while the stream has work, 0 when idle
   virtual int set_variants(const int32_t* v5, int32_t* out5) = 0;
+  virtual int set_row_launch(int launch, int* out) = 0;
   virtual int sync() = 0;
   virtual hipStream_t stream() const = 0;
   // multi-size stepping (make_fused): eligibility, the key groups must share (precision,

@@ -92,6 +92,7 @@ SIGNATURES = {
     "mhd_restart": (_I, [_P, C.c_char_p, _I]),
     "mhd_autotune": (_I, [_P, _I, C.c_char_p, _I]),
     "mhd_set_variants": (_I, [_P, _P, _P]),
+    "mhd_set_row_launch": (_I, [_P, _I, C.POINTER(_I)]),
     "mhd_set_step_pruning": (_I, [_P, _I]),
     "mhd_batch_set_step_pruning": (_I, [_P, _I]),
     "mhd_batch_autotune": (_I, [_P, _I]),

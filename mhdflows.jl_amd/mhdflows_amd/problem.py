@@ -783,6 +783,13 @@ def variants(prob, set_to=None):
     return list(out)
 
 
+def row_launch(prob, set_to=-1):
+    """Set (unless -1) and read the row launch of a right-hand side (see ``mhd_set_row_launch``)."""
+    out = C.c_int32()
+    check(lib().mhd_set_row_launch(prob._h, int(set_to), C.byref(out)))
+    return out.value
+
+
 def set_pipeline(prob, slabs):
     """Slab pipeline of each right-hand side (see ``mhd_set_pipeline``; 1 = off): the same
     results, the row kernel of one slab overlapping the y passes of another."""
