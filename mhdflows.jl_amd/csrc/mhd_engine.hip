@@ -700,6 +700,9 @@ class Engine : public EngineBase {
           for (int u = 0; u < v; ++u)
             if (col_strip<T>(n, u) == col_strip<T>(n, v)) dup = true;
           if (dup) continue;
+        } else if (!row_pairs() && (nd_any || vp_any)) {
+          best[cls] = row_var();  // negative damping and penalisation have one row launch: left alone
+          break;
         } else {
           // xrow_kernel: bit 0 plan, bit 1 swizzled LDS; skip a plan equal to a lower variant's.
           // Row pairs: skip what a lower variant launches
@@ -2144,7 +2147,7 @@ class FusedStep : public FusedBase {
       const hipError_t r = launch_small<T>(SK_PRUNE, e->rbd, e->nr_, e->phys, 1 << 20, 1, s);
       if (r != hipSuccess) return fail(E_HIP, std::string("prune marks: ") + hipGetErrorString(r));
     }
-    size_t first = 0, end = 0;  // [first, end): the first right-hand side's column and row launches
+    size_t end = 0;  // [0, end): the first right-hand side's column and row launches
     struct NoCfl {  // which choose no time step here
       FusedStep* f;
       explicit NoCfl(FusedStep* fs) : f(fs) { set(true); }
@@ -2171,7 +2174,7 @@ class FusedStep : public FusedBase {
       float sum = 0;
       for (int k = 0; k <= reps; ++k) {
         MHD_HIP(hipEventRecord(ev.a, s));
-        for (size_t i = first; i < end; ++i)
+        for (size_t i = 0; i < end; ++i)
           if (recm[0][i].type == type) MHD_TRY(launch_at(i, s));
         MHD_HIP(hipEventRecord(ev.b, s));
         MHD_HIP(hipEventSynchronize(ev.b));
