@@ -96,8 +96,9 @@ struct StepGraphs {
   StepGraphs() = default;
   StepGraphs(const StepGraphs&) = delete;
   StepGraphs& operator=(const StepGraphs&) = delete;
-  ~StepGraphs() { drop(); }
-  void drop() {
+  // their launches go to stream s: none may be queued or running when an executable is destroyed
+  void drop(hipStream_t s) {
+    if (exec[0] || exec[1]) (void)hipStreamSynchronize(s);
     for (int k = 0; k < 2; ++k) {
       if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
       if (graph[k]) (void)hipGraphDestroy(graph[k]);
@@ -174,7 +175,7 @@ class Engine : public EngineBase {
 
   ~Engine() override {
     if (st) hipStreamSynchronize(st);
-    graphs.drop();
+    graphs.drop(st);
     for (void* p : allocs) hipFree(p);
     for (void* p : force_tabs)
       if (p) hipFree(p);
@@ -1676,7 +1677,7 @@ class Engine : public EngineBase {
     return 0;
   }
   void drop_graph() {
-    graphs.drop();
+    graphs.drop(st);
     ++graph_gen_;
   }
   int forcing_done() {
@@ -1982,14 +1983,13 @@ class FusedStep : public FusedBase {
   bool multi_col = true, multi_row = true;
 
   ~FusedStep() override {
-    if (!es.empty() && es[0]->st) (void)hipStreamSynchronize(es[0]->st);
-    drop();
+    if (!es.empty()) drop();
     for (hipEvent_t e : evs)
       if (e) (void)hipEventDestroy(e);
   }
   hipStream_t stream() const { return es[0]->st; }
 
-  void drop() { graphs.drop(); }
+  void drop() { graphs.drop(stream()); }
 
   int init(const std::vector<EngineBase*>& groups) {
     for (EngineBase* b : groups) es.push_back(static_cast<Engine<T>*>(b));
