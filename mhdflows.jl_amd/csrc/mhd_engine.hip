@@ -118,8 +118,13 @@ struct StepGraphs {
       return rc;
     }
     if (e != hipSuccess) return fail(E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+    const hipError_t ie = hipGraphInstantiate(&exec[k], gr, nullptr, nullptr, 0);
+    if (ie != hipSuccess) {  // a later call captures anew
+      exec[k] = nullptr;
+      (void)hipGraphDestroy(gr);
+      return fail(E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
+    }
     graph[k] = gr;
-    MHD_HIP(hipGraphInstantiate(&exec[k], gr, nullptr, nullptr, 0));
     return 0;
   }
   // the graphs that a call of nsteps steps replays
