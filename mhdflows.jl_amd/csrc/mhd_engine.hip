@@ -348,11 +348,13 @@ class Engine : public EngineBase {
   // (memory-bound) of another.  slab_z0_/slab_z1_ bound the current slab (z1 < 0: none).
   // Default: 2 slabs for grids of 256^2 to 512^2 rows, 4 where the planes have at most 256 rows and
   // a quarter of the grid still fills the chip.  Float32 RK4 steps, ms, with 1 / 2 / 4 slabs:
-  // 256^3 2.924 / 2.906 / 2.828, 192x256x256 2.242 / 2.213 / 2.143, 128x256x512 3.193 / 3.154 / 3.062,
-  // 256x128x512 3.014 / 2.993 / 2.928 (256x256x384 alone lost: 4.432 / 4.438 / 4.462); smaller grids
-  // 96x256x256 1.166 / 1.152 / 1.219, 256x256x128 - / 1.394 / 1.402, larger planes 256x384x256
-  // - / 4.469 / 4.590, 512^3 25.06 / 24.99 / 25.01; without a magnetic field 256^3 - / 1.684 / 1.664,
-  // Float64 256^3 - / 5.512 / 5.441.  Off below (launch-bound grids) and above (1024^3: no gain).
+  // 256^3 3.139 / 3.114 / 3.094, 192x256x256 2.408 / 2.380 / 2.331, 384x256x256 4.661 / 4.629 / 4.584,
+  // 128x256x512 3.425 / 3.390 / 3.350, 256x128x512 3.227 / 3.216 / 3.189, 256x256x512 6.449 / 6.456 /
+  // 6.427; within 0.2 % 256x256x384 4.737 / 4.746 / 4.744, 256x192x384 3.578 / 3.548 / 3.555; smaller
+  // grids 96x256x256 1.277 / 1.263 / 1.330, 256x256x128 1.568 / 1.556 / 1.547, larger planes 256x384x256
+  // 4.731 / 4.744 / 4.821, 512^3 26.46 / 26.53 / 26.46; without a magnetic field 256^3 1.908 / 1.873 /
+  // 1.875, Float64 256^3 5.871 / 5.795 / 5.743.  Off below (launch-bound grids) and above (1024^3: no
+  // gain).
   int pipe_ = 1;
   int slab_z0_ = 0, slab_z1_ = -1;
   // slab boundaries of the pipeline for row variant rvar (each slab starts on a whole row
@@ -479,9 +481,10 @@ class Engine : public EngineBase {
     return rhs_row_variant(row_pairs() ? pair_var : xrow_var);
   }
   int rhs_row_variant(int v) const {
-    // xrow_kernel's swizzled LDS index from 128 points (Float64: 64) up.  RK4 steps with a static force,
-    // ms, plain / swizzled: Float32 96^3 0.362 / 0.370, 128^3 0.522 / 0.508, 192^3 1.465 / 1.415, 256^3 3.67 /
-    // 3.39; Float64 48^3 0.273 / 0.276, 64^3 0.293 / 0.279, 128^3 0.932 / 0.897.  The bits do not depend on it.
+    // xrow_kernel's swizzled LDS index from 128 points (Float64: 64) up; negative damping and
+    // penalisation have variant 0 only.  RK4 steps with a static force, ms, plain / swizzled: Float32
+    // 96^3 0.362 / 0.370, 128^3 0.522 / 0.508, 192^3 1.465 / 1.415, 256^3 3.67 / 3.39; Float64 48^3 0.273 /
+    // 0.276, 64^3 0.293 / 0.279, 128^3 0.932 / 0.897.  The bits do not depend on it.
     if (!row_pairs()) return v ^ (g.nx >= (sizeof(T) == 8 ? 64 : 128) ? 2 : 0);
     const bool f64 = sizeof(T) == 8;
     const int64_t pairs = (int64_t)g.ny * g.nz / 2;
