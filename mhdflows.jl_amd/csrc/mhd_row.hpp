@@ -78,20 +78,21 @@ MHD_ROWPLAN2_B(768, 1, 6, 4, 4, 8, 6)
 MHD_ROWPLAN2_B(1024, 1, 16, 16, 16, 4)
 #undef MHD_ROWPLAN2_B
 // The plan a row launch uses unless its variant asks for the other one.  Six fields (MHD) of three
-// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 221 (two); up to 768
-// points the waves are worth more than the shorter sequence of passes, at 1024 the passes are.  us a
-// launch of a dealiased step, plan 0 / plan 1: Float32 192^3 95 / 90, 256^3 197 / 191, 384x128x192
-// 149 / 132, 1024x128x64 129 / 157 (against the rule 128^3 28.5 / 29.4, 512x256x128 203 / 214); Float64
-// 128^3 53 / 50, 192^3 206 / 188, 256x256x128 213 / 189.  Lengths with a factor 3 in six values of
-// radix-2 passes and a last one of 6 took 172 where 384x128x192 took 128 (768x256x192 719 with twelve
-// values / 647; Float64 192^3 240 / 183, 384x128x192 315 / 291).  Three fields (HD) leave both plans
-// their waves: fewer values only where launches are too small to fill the chip, at 384 points with
-// their three passes (Float32 81 / 68; Float64 165 / 113) and at 768 in Float64, where twelve values
-// take the waves all the same (617 / 525, Float32 261 / 288); otherwise plan 0 (256^3 96 / 99,
-// 512x256x128 84 / 100).
+// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 221 (two); below 512
+// points the waves are worth more than the shorter sequence of passes, at 1024 the passes are, and
+// at 768 Float64 the six values of plan 1 cost more than the twelve of plan 0.  RK4 steps, ms, plan
+// 0 / plan 1: Float32 128x256x128 0.899 / 0.866, 192x256x128 1.214 / 1.166, 256x256x128 1.679 / 1.603,
+// 384x256x128 2.607 / 2.526, 512x64x64 0.420 / 0.438, 512^3 26.19 / 26.58, 768x128x128 2.59 / 2.51,
+// 768x256x256 10.48 / 10.16, 1024x128x128 3.21 / 3.49; Float64 128x256x128 1.712 / 1.638, 192x256x128
+// 2.521 / 2.424, 256x256x128 3.265 / 3.131, 512x256x256 12.65 / 12.46, 768x128x128 4.83 / 8.63,
+// 1024x128x128 6.42 / 12.03.  Three fields (HD) leave both plans their waves: fewer values only where
+// launches are too small to fill the chip and at 384 points with their three passes (Float32
+// 384x256x128 1.440 / 1.387, Float64 2.959 / 2.661); otherwise plan 0 (Float32 192x256x128 0.704 /
+// 0.718, 512x128x128 0.854 / 0.905, 768x128x128 1.374 / 1.409; Float64 512x128x128 1.700 / 1.780,
+// 768x128x128 2.83 / 4.74).
 inline int rowpair_plan(int nx, int phys, bool f64) {
-  if (phys == PHYS_MHD) return nx < 1024 ? 1 : 0;
-  return nx <= 96 || nx == 384 || (nx == 768 && f64) ? 1 : 0;
+  if (phys == PHYS_MHD) return nx < 512 || nx == (f64 ? 512 : 768) ? 1 : 0;
+  return nx <= 96 || nx == 384 ? 1 : 0;
 }
 // values a thread holds, for host-side launch shapes
 inline int rowpair_E(int nx, int plan) {
@@ -109,21 +110,22 @@ inline int rowpair_E(int nx, int plan) {
 // took 22.7 and 24.4 us at 96^3 for 21.7.
 constexpr int ROW_TEAM = 2, ROW_TEAM_HALF = 3;
 inline bool rowteam_length(int nx) { return nx <= 256; }
-// The team that a whole launch over `pairs` row pairs takes, 0 for none.  The waves of a plain launch each run 15 (HD:
-// 9) transforms one after the other; with less than about two of them a SIMD the launch takes as
-// long as one wave does, and teams shorten that.  us a launch, plain / a wave per product / three
-// waves, by the waves of the plain launch: Float32 32^3 (64) 12.0 / 8.0 / 9.0, 48^3 (288) 12.9 / 9.4 /
-// 10.2, 64^3 (512) 14.1 / 10.7 / 11.2, 128x64x64 (1024) 17.8 / 16.6 / 14.9, 256x64x64 (2048) 21.4 /
-// 26.9 / 22.0, 96^3 (2304) 23.1 / 29.7 / 21.7, 192x96x64 (3072) 25.6 / 37.5 / 26.5; Float64 32^3 13.8 /
-// 9.0 / 9.9, 48^3 14.8 / 12.8 / 11.6, 64^3 16.6 / 15.2 / 13.8, 96^3 37.1 / 47.6 / 31.1, 128x96x64 (1536)
-// 25.1 / 37.8 / 28.2.  Without a magnetic field:
-// Float32 32^3 9.5 / 7.0 / 7.4, 64^3 10.4 / 8.6 / 8.7, 128x96x64 16.0 / 14.1 / 13.3, 128^3 (4096)
-// 21.1 / 27.1 / 22.2; Float64 64^3 11.9 / 10.2 / 10.1, 128x96x64 20.2 / 22.5 / 18.9.
+// The team that a whole launch over `pairs` row pairs takes, 0 for none.  The waves of a plain
+// launch each run 15 (HD: 9) transforms one after the other; with less than about two of them a SIMD
+// the launch takes as long as one wave does, and teams shorten that.  us a launch, plain / a wave per
+// product / three waves, by the waves of the plain launch: Float32 32^3 (64) 12.0 / 8.0 / 9.0, 48^3
+// (288) 12.9 / 9.4 / 10.2, 64^3 (512) 14.1 / 10.7 / 11.2, 128x64x64 (1024) 17.8 / 16.6 / 14.9,
+// 256x64x64 (2048) 21.4 / 26.9 / 22.0, 96^3 (2304) 23.1 / 29.7 / 21.7, 192x96x64 (3072) 25.6 / 37.5 /
+// 26.5; Float64 32^3 13.8 / 9.0 / 9.9, 48^3 14.8 / 12.8 / 11.6, 64^3 16.6 / 15.2 / 13.8, 96^3 37.1 / 47.6 /
+// 31.1, 128x96x64 (1536) 25.1 / 37.8 / 28.2, an RK4 step of 192x64x64 (2048) 383 plain / 396 three waves.
+// Without a magnetic field: Float32 32^3 9.5 / 7.0 / 7.4, 64^3 10.4 / 8.6 / 8.7, 128x96x64 16.0 / 14.1 /
+// 13.3, 128^3 (4096) 21.1 / 27.1 / 22.2; Float64 64^3 11.9 / 10.2 / 10.1, 128x96x64 20.2 / 22.5 / 18.9.
 inline int rowpair_team(int nx, int phys, bool f64, int64_t pairs) {
   if (!rowteam_length(nx)) return 0;
   const int64_t waves = pairs * (nx / rowpair_E(nx, 1)) / 64;
-  if (waves < (f64 && phys == PHYS_MHD ? 384 : 768)) return ROW_TEAM;
-  return waves < (nx % 3 && (f64 || phys == PHYS_MHD) ? 1280 : 2560) ? ROW_TEAM_HALF : 0;
+  if (waves < (f64 && phys == PHYS_MHD ? 192 : 768)) return ROW_TEAM;
+  const bool early = nx % 3 ? f64 || phys == PHYS_MHD : f64 && phys == PHYS_MHD && nx > 96;
+  return waves < (early ? 1280 : 2560) ? ROW_TEAM_HALF : 0;
 }
 // The plan of a grid of `pairs` row pairs: plan 1 where one run is a team.  It does not depend on the
 // number of runs, so a run ends with the same bits alone and beside others.

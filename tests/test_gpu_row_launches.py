@@ -52,3 +52,11 @@ def test_what_sets_and_ends_a_launch():
     assert M.row_launch(p) == -1
     with pytest.raises(M.MHDError):
         M.row_launch(p, 1)
+
+
+# 768-point Float64 rows are 1.8 times as slow with the six values a thread of plan 1
+@pytest.mark.parametrize("nx,T,mhd,launch", [(768, np.float64, True, 0), (768, np.float64, False, 0),
+                                             (768, np.float32, True, 1), (512, np.float32, True, 0)])
+def test_choice_for_long_rows(nx, T, mhd, launch):
+    p = M.Problem("MI355X", nx=nx, ny=64, nz=64, B_field=mhd, T=T, dt=1e-3)
+    assert M.row_launch(p) == launch
