@@ -477,9 +477,11 @@ class Engine : public EngineBase {
     return row_pairs() ? rowpair_rows_per_block(g.nx, var) : row_rows_per_block<T>(g.nx, var);
   }
   int rhs_row_variant() const {
-    if (row_pairs() && row_launch_ >= 0) return row_launch_;
+    if (row_pairs() && row_launch_ >= 0) return without_teams(row_launch_);
     return rhs_row_variant(row_pairs() ? pair_var : xrow_var);
   }
+  // multi-size launches have the teams' plan without teams
+  int without_teams(int r) const { return rec_ && rec_multi_ && r >= ROW_TEAM ? 1 : r; }
   int rhs_row_variant(int v) const {
     // xrow_kernel's swizzled LDS index from 128 points (Float64: 64) up; negative damping and
     // penalisation have variant 0 only.  RK4 steps with a static force, ms, plain / swizzled: Float32
@@ -492,7 +494,7 @@ class Engine : public EngineBase {
     const int choice = rowpair_choice(g.nx, phys, f64, pairs, nr_);
     int r = v >= 2 && rowteam_length(g.nx) ? v : choice;
     if (v == 1) r = choice >= ROW_TEAM ? plan : plan ^ 1;
-    return rec_ && rec_multi_ && r >= ROW_TEAM ? 1 : r;  // multi-size launches have the plan without teams
+    return without_teams(r);
   }
   RowArgs rhs_row_args(int var) const { return row_args_of(rhs_rows_per_block(var)); }
   // the other row launches: xrow_kernel, variant 0
