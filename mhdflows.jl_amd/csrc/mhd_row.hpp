@@ -78,9 +78,9 @@ MHD_ROWPLAN2_B(768, 1, 6, 4, 4, 8, 6)
 MHD_ROWPLAN2_B(1024, 1, 16, 16, 16, 4)
 #undef MHD_ROWPLAN2_B
 // The plan a row launch uses unless its variant asks for the other one.  Six fields (MHD) of three
-// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 221 (two); below 512
+// or four values a thread fit 128 VGPRs (Float32: four waves a SIMD), of eight 211 (two); below 512
 // points the waves are worth more than the shorter sequence of passes, at 1024 the passes are, and
-// at 768 Float64 the six values of plan 1 cost more than the twelve of plan 0.  RK4 steps, ms, plan
+// at 768 Float64 plan 1 is compiled with 144 B of scratch a lane.  RK4 steps, ms, plan
 // 0 / plan 1: Float32 128x256x128 0.899 / 0.866, 192x256x128 1.214 / 1.166, 256x256x128 1.679 / 1.603,
 // 384x256x128 2.607 / 2.526, 512x64x64 0.420 / 0.438, 512^3 26.19 / 26.58, 768x128x128 2.59 / 2.51,
 // 768x256x256 10.48 / 10.16, 1024x128x128 3.21 / 3.49; Float64 128x256x128 1.712 / 1.638, 192x256x128
